@@ -645,6 +645,21 @@ DEVI int tx_quant1(int v, bool dc, int dcQ, int acQ, float rDc, float rAc, int d
   return v < 0 ? -level : level;
 }
 
+/* tx_quant1 for the transforms up to 16x16 (denominator 1), whose
+ * coefficients are bounded: |residual| <= 255 and matrix rows with an L1
+ * norm below 1.49e6 leave row outputs below 5800 and column sums below
+ * 2^33.1, so |v| < 2^33.1 * 2^6 * sqrt(2) / 2^20 < 2^20, and with
+ * q <= 1828 t = (|v| + 6.5 q) / 16 < 2^17: the reciprocal form always
+ * applies and the level stays below 0xFFFF (q >= 4). */
+DEVI int tx_quant_small(int v, int q, int add, float rq) {
+  const int t = (d_abs(v) + add) >> 4;
+  const int l = tx_qdiv(t, q, rq);
+  return v < 0 ? -l : l;
+}
+DEVI int tx_quant_add(int q, bool dc) { return (q * (dc ? 26 : 22)) >> 2; }
+/* s * 2^sh / 2^20 rounded to nearest, halves away from zero. */
+DEVI int tx_round_col(long long s, int sh) { return (int)((s + ((1ll << (19 - sh)) + (s >> 63))) >> (20 - sh)); }
+
 /* One wave's forward transform of a (1 << LH) x (1 << LW) block, both
  * lengths at most 16, with the sizes known at compile time: every LDS
  * access is a fixed offset from a per-lane base, so the loads of a sum issue
@@ -682,14 +697,19 @@ DEVI int sfwd(const lds_i32 *resid, int rs, lds_i32 *tmp, lds_i32 *coef, const l
       long long s = 0;
 #pragma unroll
       for (int i = 0; i < H; i++) s += (long long)m[i] * col[i];
-      s *= (1ll << sh);
-      if constexpr (RECT) s = ((s + 2048) >> 12) * 5793;
-      const int v = (int32_t)(s >= 0 ? (s + (1ll << 19)) >> 20 : -((-s + (1ll << 19)) >> 20));
+      int v;
+      if constexpr (RECT) {
+        s *= (1ll << sh);
+        v = tx_round_col(((s + 2048) >> 12) * 5793, 0);
+      } else {
+        v = tx_round_col(s, sh);
+      }
       /* QUANT: the level at once (sizes up to 16 have no dequantiser
        * denominator), and the eob: 1 + the largest scan position (iscan)
        * of a non-zero level */
       if constexpr (QUANT) {
-        const int lv = tx_quant1(v, k == 0, dcQ, acQ, rDc, rAc, 1);
+        const int lv = tx_quant_small(v, k == 0 ? dcQ : acQ, k == 0 ? tx_quant_add(dcQ, true) : tx_quant_add(acQ, false),
+                                      k == 0 ? rDc : rAc);
         coef[k] = lv;
         if (lv) eob = d_max(eob, iscan[k] + 1);
       } else {

@@ -123,6 +123,7 @@ DEVI uint8_t *tile_ptr(int k, int plane, int miRow, int miCol, int &S) {
 DEVI int lane_xor1(int v) { return dpp_t<DPP_QX1>(v); }
 DEVI int lane_xor2(int v) { return dpp_t<DPP_QX2>(v); }
 DEVI int lane_xor4(int v) { return dpp_t<DPP_HMIRROR>(dpp_t<0x1B>(v)); } /* 7 - i of 3 - i within the quad */
+DEVI int lane_xor8(int v) { return dpp_t<DPP_MIRROR>(dpp_t<DPP_HMIRROR>(v)); } /* 15 - i of 7 - i within the half row */
 /* a[j] of lane i <-> a[i] of lane j within each group of N lanes. */
 template <int N>
 DEVI void lane_transpose(int32_t (&a)[N], int r) {
@@ -132,10 +133,11 @@ DEVI void lane_transpose(int32_t (&a)[N], int r) {
 #pragma unroll
     for (int i = 0; i < N; i++) {
       if (i & b) continue;
-      const int32_t x = hi ? a[i] : a[i | b];
-      const int32_t y = b == 1 ? lane_xor1(x) : b == 2 ? lane_xor2(x) : lane_xor4(x);
-      if (hi) a[i] = y;
-      else a[i | b] = y;
+      const int32_t x0 = a[i], x1 = a[i | b], x = hi ? x0 : x1;
+      const int32_t y = b == 1 ? lane_xor1(x) : b == 2 ? lane_xor2(x) : b == 4 ? lane_xor4(x) : lane_xor8(x);
+      /* selects of values: a store to one of two elements would put the array in scratch memory */
+      a[i] = hi ? y : x0;
+      a[i | b] = hi ? x1 : y;
     }
   }
 }
@@ -154,80 +156,23 @@ DEVI int lane_group_max(int v) {
   return v;
 }
 
-/* The transform types of a 4x4 (LN 2) or 8x8 (LN 3) intra luma block side by
- * side on one wave: candidate type k of the list `types` (nc <= 8 nibbles,
- * none of them flipped) on lanes k * N .. k * N + N - 1, one lane per row or
- * column. A lane keeps its row or column in registers through the residual,
- * the two forward passes, the quantiser, the dequantiser and the two inverse
- * passes; rows and columns change place by lane swaps, so the search has no
- * LDS round trip besides its tables. Same values as tx_eval of each type,
- * then the first minimum: the levels go to lev (stride N), the
- * reconstruction into px (row stride S) at (x, y). Every lane of the wave
- * calls it; *type / *eob / the cost are the same in every lane.
- * Bound by one wave's issue rate (a serial chain of about 900 instructions
- * for 8x8, 400 for 4x4): the eight waves of tx_eval took 11.7k cycles for an
- * 8x8 and 9.7k for a 4x4, with five barriers around them. */
+/* Row, column and scan kind of a type (row_kind, col_kind, scan_kind), two
+ * bits per type, for types that differ between lanes. */
+constexpr uint32_t kind_table(int which) {
+  const int row[16] = {0, 0, 1, 1, 0, 1, 1, 1, 1, 2, 2, 0, 2, 1, 2, 1};
+  const int col[16] = {0, 1, 0, 1, 1, 0, 1, 1, 1, 2, 0, 2, 1, 2, 1, 2};
+  const int scan[16] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 1, 2, 1, 2, 1, 2};
+  uint32_t v = 0;
+  for (int t = 0; t < 16; t++) v |= (uint32_t)(which == 0 ? row[t] : which == 1 ? col[t] : scan[t]) << (2 * t);
+  return v;
+}
+
+/* The inverse transform of a square block on lanes 0 .. N - 1 of a wave (and
+ * alike on the other groups of N lanes): lane r enters with row r of the
+ * dequantised coefficients in T and leaves with row r of the residual. */
 template <int LN>
-DEVI long long wave_tx_search(const Mav1FrameParams &fp, const uint8_t *spx, int SS, uint8_t *px, int S, int x, int y,
-                              unsigned long long types, int nc, int32_t *lev_, int *typeOut, int *eobOut) {
-  constexpr int N = 1 << LN, RS = LN == 3 ? 1 : 0; /* RS: Transform_Row_Shift */
-  typedef __attribute__((address_space(3))) uint32_t lds_u32;
-  const int lane = d_local(threadIdx.x & 63), r = lane & (N - 1), gi = lane >> LN;
-  nc = d_uni(nc);
-  const int t = (int)(types >> (4 * (gi < nc ? gi : 0))) & 15;
-  const int rk = row_kind(t), ck = col_kind(t);
-  const int dcQ = fp.dc_q[0], acQ = fp.ac_q[0];
-  const float rDc = gL.qrcp[0][0], rAc = gL.qrcp[0][1];
-  /* row r of the source and the prediction */
-  uint32_t sw[N / 4], pw[N / 4];
-  const lds_u32 *sp = (const lds_u32 *)(spx + (y + r) * SS + x);
-  lds_u32 *pp = (lds_u32 *)(px + (y + r) * S + x);
-#pragma unroll
-  for (int j = 0; j < N / 4; j++) {
-    sw[j] = sp[j];
-    pw[j] = pp[j];
-  }
-  int32_t d[N];
-#pragma unroll
-  for (int j = 0; j < N; j++) d[j] = (int)((sw[j >> 2] >> (8 * (j & 3))) & 255) - (int)((pw[j >> 2] >> (8 * (j & 3))) & 255);
-  /* forward rows, then columns (lane r holds column r) and the quantiser */
-  const lds_i32 *Mh = lds(gL.smats) + smat_off(rk, LN), *Mv = lds(gL.smats) + smat_off(ck, LN);
-  int32_t T[N];
-#pragma unroll
-  for (int k = 0; k < N; k++) {
-    int s = 0;
-#pragma unroll
-    for (int j = 0; j < N; j++) s += __mul24(d[j], Mh[k * N + j]);
-    T[k] = (s + 32768) >> 16;
-  }
-  lane_transpose<N>(T, r);
-  const lds_i16 *is = (const lds_i16 *)(gL.iscans + scan_kind(t) * SCAN_SMALL + (LN == 2 ? 0 : 16));
-  int32_t q[N];
-  int pos[N], eob = 0;
-#pragma unroll
-  for (int k = 0; k < N; k++) {
-    long long s = 0;
-#pragma unroll
-    for (int i = 0; i < N; i++) s += (long long)Mv[k * N + i] * T[i];
-    s *= (1ll << (RS + 4));
-    const int v = (int32_t)(s >= 0 ? (s + (1ll << 19)) >> 20 : -((-s + (1ll << 19)) >> 20));
-    q[k] = tx_quant1(v, k == 0 && r == 0, dcQ, acQ, rDc, rAc, 1);
-    pos[k] = is[k * N + r];
-    if (q[k]) eob = d_max(eob, pos[k] + 1);
-  }
-  eob = lane_group_max<N>(eob);
-  /* the rate (tx_bits) and the dequantised levels */
-  int bits = 0;
-#pragma unroll
-  for (int k = 0; k < N; k++) {
-    const int l = d_abs(q[k]);
-    if (pos[k] < eob) bits += l ? 8 * (2 + 2 * d_floorlog2((unsigned)l)) : 6;
-    const int ad = __mul24(l, (k == 0 && r == 0) ? dcQ : acQ) & 0xFFFFFF;
-    T[k] = d_clip(-(1 << 15), (1 << 15) - 1, q[k] < 0 ? -ad : ad);
-  }
-  bits = lane_group_sum<N>(bits);
-  bits = eob ? 48 + 16 * d_floorlog2((unsigned)eob + 1) + bits : 8;
-  lane_transpose<N>(T, r);
+DEVI void lane_itx(int32_t (&T)[1 << LN], int rk, int ck, int r) {
+  constexpr int N = 1 << LN, RS = LN - 2; /* Transform_Row_Shift of 4x4, 8x8, 16x16 */
   if (rk == 0) t_idct<LN>(T, 16);
   else if (rk == 1) t_1d<1, LN>(T, 16);
   else t_identity<LN>(T);
@@ -238,7 +183,140 @@ DEVI long long wave_tx_search(const Mav1FrameParams &fp, const uint8_t *spx, int
   else if (ck == 1) t_1d<1, LN>(T, 16);
   else t_identity<LN>(T);
   lane_transpose<N>(T, r);
-  /* back on rows: the reconstruction and its SSE */
+#pragma unroll
+  for (int j = 0; j < N; j++) T[j] = d_round2(T[j], 4);
+}
+typedef __attribute__((address_space(3))) uint32_t lds_u32;
+/* One wave's reconstruction of a square block (tx_recon_small without a
+ * flip): the levels q (LDS, stride N) dequantised, inverse transformed with
+ * rows and columns changing place by lane swaps and added to px, whole words
+ * at a time. Bound by the wave's serial chain: two LDS round trips fewer than
+ * two passes over LDS with byte-wise adds, 2.4k cycles for a luma block of a
+ * 1080p key frame instead of 3.1k. */
+template <int LN>
+DEVI void wave_recon(const int32_t *q_, int rk, int ck, int dcQ, int acQ, uint8_t *px, int S, int x, int y) {
+  constexpr int N = 1 << LN;
+  const int lane = d_local(threadIdx.x & 63), r = lane & (N - 1);
+  const lds_i32 *q = lds(q_) + r * N;
+  lds_u32 *pp = (lds_u32 *)(px + (y + r) * S + x);
+  uint32_t pw[N / 4];
+#pragma unroll
+  for (int j = 0; j < N / 4; j++) pw[j] = pp[j];
+  int32_t T[N];
+#pragma unroll
+  for (int j = 0; j < N; j++) {
+    const int l = q[j], ad = __mul24(d_abs(l), (j == 0 && r == 0) ? dcQ : acQ) & 0xFFFFFF;
+    T[j] = d_clip(-(1 << 15), (1 << 15) - 1, l < 0 ? -ad : ad);
+  }
+  lane_itx<LN>(T, rk, ck, r);
+  uint32_t rw[N / 4];
+#pragma unroll
+  for (int j = 0; j < N / 4; j++) rw[j] = 0;
+#pragma unroll
+  for (int j = 0; j < N; j++) {
+    const int sh = 8 * (j & 3);
+    rw[j >> 2] |= (uint32_t)d_clip1((int)((pw[j >> 2] >> sh) & 255) + T[j]) << sh;
+  }
+  if (lane < N) {
+#pragma unroll
+    for (int j = 0; j < N / 4; j++) pp[j] = rw[j];
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+/* tx_recon_small of an intra block (no flipped types). */
+DEVI void wave_recon_any(const TxCtx &c, const int32_t *q, int32_t *res, int txSz, int type, int dcQ, int acQ,
+                         uint8_t *px, int S, int x, int y) {
+  txSz = d_uni(txSz);
+  type = d_uni(type);
+  const int rk = row_kind(type), ck = col_kind(type);
+  if (txSz == TX_4X4) wave_recon<2>(q, rk, ck, dcQ, acQ, px, S, x, y);
+  else if (txSz == TX_8X8) wave_recon<3>(q, rk, ck, dcQ, acQ, px, S, x, y);
+  else if (txSz == TX_16X16) wave_recon<4>(q, rk, ck, dcQ, acQ, px, S, x, y);
+  else tx_recon_small(c, q, res, SRS, txSz, type, dcQ, acQ, px, S, x, y);
+}
+
+/* The transform types of a 4x4 (LN 2) or 8x8 (LN 3) intra luma block side by
+ * side on one wave: candidate type k of the list `types` (nc <= 8 nibbles,
+ * none of them flipped) on lanes k * N .. k * N + N - 1, one lane per row or
+ * column. A lane keeps its row or column in registers through the residual,
+ * the two forward passes, the quantiser, the dequantiser and the two inverse
+ * passes; rows and columns change place by lane swaps, so the search has no
+ * LDS round trip besides its tables. Same values as tx_eval of each type,
+ * then the first minimum: the levels go to lev (stride N), the
+ * reconstruction into px (row stride S) at (x, y). Every lane of the wave
+ * calls it; *type / *eob / the cost are the same in every lane.
+ * Bound by one wave's issue rate (a serial chain): 8.6k cycles for an 8x8 and
+ * 3.1k for a 4x4; the eight waves of tx_eval took 11.7k and 9.7k, with five
+ * barriers around them, and this search with its passes through LDS 17k and
+ * 7.9k. */
+template <int LN>
+DEVI long long wave_tx_search(const Mav1FrameParams &fp, const uint8_t *spx, int SS, uint8_t *px, int S, int x, int y,
+                              unsigned long long types, int nc, int32_t *lev_, int *typeOut, int *eobOut) {
+  constexpr int N = 1 << LN, SH = LN == 3 ? 5 : 4; /* Transform_Row_Shift + 4 */
+  constexpr uint32_t RK = kind_table(0), CK = kind_table(1), SK = kind_table(2);
+  const int lane = d_local(threadIdx.x & 63), r = lane & (N - 1), gi = lane >> LN;
+  nc = d_uni(nc);
+  const int t = (int)(types >> (4 * (gi < nc ? gi : 0))) & 15;
+  const int rk = (RK >> (2 * t)) & 3, ck = (CK >> (2 * t)) & 3;
+  const int dcQ = fp.dc_q[0], acQ = fp.ac_q[0], addDc = tx_quant_add(dcQ, true), addAc = tx_quant_add(acQ, false);
+  const float rDc = gL.qrcp[0][0], rAc = gL.qrcp[0][1];
+  /* row r of the source and the prediction */
+  uint32_t sw[N / 4], pw[N / 4];
+  const lds_u32 *sp = (const lds_u32 *)(spx + (y + r) * SS + x);
+  lds_u32 *pp = (lds_u32 *)(px + (y + r) * S + x);
+#pragma unroll
+  for (int j = 0; j < N / 4; j++) {
+    sw[j] = sp[j];
+    pw[j] = pp[j];
+  }
+  const lds_i16 *is = (const lds_i16 *)(gL.iscans + ((SK >> (2 * t)) & 3) * SCAN_SMALL + (LN == 2 ? 0 : 16));
+  int pos[N];
+#pragma unroll
+  for (int k = 0; k < N; k++) pos[k] = is[k * N + r];
+  int32_t d[N];
+#pragma unroll
+  for (int j = 0; j < N; j++) d[j] = (int)((sw[j >> 2] >> (8 * (j & 3))) & 255) - (int)((pw[j >> 2] >> (8 * (j & 3))) & 255);
+  /* forward rows, then columns (lane r holds column r) and the quantiser */
+  const lds_i32 *Mh = lds(gL.smats) + rk * 336 + (LN == 2 ? 0 : 16), *Mv = lds(gL.smats) + ck * 336 + (LN == 2 ? 0 : 16);
+  int32_t T[N];
+#pragma unroll
+  for (int k = 0; k < N; k++) {
+    int s = 32768;
+#pragma unroll
+    for (int j = 0; j < N; j++) s += __mul24(d[j], Mh[k * N + j]);
+    T[k] = s >> 16;
+  }
+  lane_transpose<N>(T, r);
+  int32_t q[N];
+  int eob = 0;
+#pragma unroll
+  for (int k = 0; k < N; k++) {
+    long long s = 0;
+#pragma unroll
+    for (int i = 0; i < N; i++) s += (long long)Mv[k * N + i] * T[i];
+    const bool dc = k == 0 && r == 0;
+    q[k] = tx_quant_small(tx_round_col(s, SH), dc ? dcQ : acQ, dc ? addDc : addAc, dc ? rDc : rAc);
+    eob = d_max(eob, q[k] ? pos[k] + 1 : 0);
+  }
+  eob = lane_group_max<N>(eob);
+  /* the rate (tx_bits) and the dequantised levels */
+  int bits = 0;
+#pragma unroll
+  for (int k = 0; k < N; k++) {
+    const int l = d_abs(q[k]);
+    /* 8 (2 + 2 floor(log2 l)) = 16 (32 - clz(l)); 6 for a zero */
+    const int lb = l ? 16 * (32 - __clz(l)) : 6;
+    bits += pos[k] < eob ? lb : 0;
+    const int ad = __mul24(l, (k == 0 && r == 0) ? dcQ : acQ) & 0xFFFFFF;
+    T[k] = d_clip(-(1 << 15), (1 << 15) - 1, q[k] < 0 ? -ad : ad);
+  }
+  bits = lane_group_sum<N>(bits);
+  bits = eob ? 48 + 16 * d_floorlog2((unsigned)eob + 1) + bits : 8;
+  lane_transpose<N>(T, r);
+  lane_itx<LN>(T, rk, ck, r);
+  /* on rows: the reconstruction and its SSE */
   int e = 0;
   uint32_t rw[N / 4];
 #pragma unroll
@@ -246,28 +324,27 @@ DEVI long long wave_tx_search(const Mav1FrameParams &fp, const uint8_t *spx, int
 #pragma unroll
   for (int j = 0; j < N; j++) {
     const int sh = 8 * (j & 3);
-    const int v = d_clip1((int)((pw[j >> 2] >> sh) & 255) + d_round2(T[j], 4));
+    const int v = d_clip1((int)((pw[j >> 2] >> sh) & 255) + T[j]);
     const int dd = (int)((sw[j >> 2] >> sh) & 255) - v;
-    e += dd * dd;
+    e += __mul24(dd, dd);
     rw[j >> 2] |= (uint32_t)v << sh;
   }
   e = lane_group_sum<N>(e);
   const long long cost = (long long)e * 16 + (long long)fp.lambda * bits / 8;
-  /* the first minimum over the candidates */
-  long long best = 0;
-  int win = 0;
-#pragma unroll 1
-  for (int k = 0; k < nc; k++) {
-    const unsigned lo = __builtin_amdgcn_readlane((int)(unsigned)cost, k * N);
-    const int hi = __builtin_amdgcn_readlane((int)(cost >> 32), k * N);
+  /* the first minimum over the candidates: cost < 2^40, so the candidate
+   * index fits beside it */
+  long long best = LLONG_MAX;
+  const long long key = gi < nc ? cost << 4 | gi : LLONG_MAX;
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    const unsigned lo = __builtin_amdgcn_readlane((int)(unsigned)key, k * N);
+    const int hi = __builtin_amdgcn_readlane((int)(key >> 32), k * N);
     const long long c = (long long)(((unsigned long long)(unsigned)hi << 32) | lo);
-    if (k == 0 || c < best) {
-      best = c;
-      win = k;
-    }
+    best = c < best ? c : best;
   }
+  const int win = (int)best & 15;
   const int we = __builtin_amdgcn_readlane(eob, win * N);
-  *typeOut = we > 0 ? __builtin_amdgcn_readlane(t, win * N) : DCT_DCT;
+  *typeOut = we > 0 ? (int)(types >> (4 * win)) & 15 : DCT_DCT;
   *eobOut = we;
   if (gi == win) {
     lds_i32 *lev = lds(lev_);
@@ -279,7 +356,68 @@ DEVI long long wave_tx_search(const Mav1FrameParams &fp, const uint8_t *spx, int
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  return best;
+  return best >> 4;
+}
+
+/* The single type of a 4x4 block on one wave (its four rows on the lanes of
+ * each group of four): levels to lev, the reconstruction into px; returns
+ * the eob. Same values as tx_eval and tx_recon_small. */
+DEVI int wave_tx4(const Mav1FrameParams &fp, int plane, const uint8_t *spx, int SS, uint8_t *px, int S, int x, int y,
+                  int t, int32_t *lev_) {
+  const int lane = d_local(threadIdx.x & 63), r = lane & 3;
+  const int rk = row_kind(t), ck = col_kind(t);
+  const int dcQ = fp.dc_q[plane], acQ = fp.ac_q[plane];
+  const float rDc = gL.qrcp[plane][0], rAc = gL.qrcp[plane][1];
+  const uint32_t sw = *(const lds_u32 *)(spx + (y + r) * SS + x);
+  lds_u32 *pp = (lds_u32 *)(px + (y + r) * S + x);
+  const uint32_t pw = *pp;
+  const lds_i32 *Mh = lds(gL.smats) + rk * 336, *Mv = lds(gL.smats) + ck * 336;
+  int32_t d[4], T[4], q[4];
+#pragma unroll
+  for (int j = 0; j < 4; j++) d[j] = (int)((sw >> (8 * j)) & 255) - (int)((pw >> (8 * j)) & 255);
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    int s = 32768;
+#pragma unroll
+    for (int j = 0; j < 4; j++) s += __mul24(d[j], Mh[k * 4 + j]);
+    T[k] = s >> 16;
+  }
+  lane_transpose<4>(T, r);
+  const lds_i16 *is = (const lds_i16 *)(gL.iscans + scan_kind(t) * SCAN_SMALL);
+  int eob = 0;
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    long long s = 0;
+#pragma unroll
+    for (int i = 0; i < 4; i++) s += (long long)Mv[k * 4 + i] * T[i];
+    const bool dc = k == 0 && r == 0;
+    q[k] = tx_quant_small(tx_round_col(s, 4), dc ? dcQ : acQ, dc ? tx_quant_add(dcQ, true) : tx_quant_add(acQ, false),
+                          dc ? rDc : rAc);
+    eob = d_max(eob, q[k] ? is[k * 4 + r] + 1 : 0);
+  }
+  eob = d_uni(lane_group_max<4>(eob));
+  lds_i32 *lev = lds(lev_);
+  if (lane < 4) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) lev[k * 4 + r] = q[k];
+  }
+  if (eob > 0) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const int ad = __mul24(d_abs(q[k]), (k == 0 && r == 0) ? dcQ : acQ) & 0xFFFFFF;
+      T[k] = d_clip(-(1 << 15), (1 << 15) - 1, q[k] < 0 ? -ad : ad);
+    }
+    lane_transpose<4>(T, r);
+    lane_itx<2>(T, rk, ck, r);
+    uint32_t rw = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) rw |= (uint32_t)d_clip1((int)((pw >> (8 * j)) & 255) + T[j]) << (8 * j);
+    if (lane < 4) *pp = rw;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  return eob;
 }
 
 /* ---- intra prediction of one transform block with the normative edge
@@ -409,6 +547,120 @@ DEVI void intra_tx_predict(const TxCtx &c, uint8_t *px, int S, int sx, int sy, i
     px[(sy + i) * S + sx + j] = (uint8_t)intra_px(im, A, Lc, i, j);
   }
   tx_sync(c);
+}
+
+/* intra_tx_predict of a block of at most 8x8 by one wave: the edges stay in
+ * registers, the row above on lanes 0 .. 31 (lane l: sample l - 1) and the
+ * column left on lanes 32 .. 63, so that both are filtered and upsampled by
+ * the same instructions, with lane permutes instead of copies through LDS.
+ * Only the finished edges go to LDS (eA / eL), for the predictors that index
+ * them. Same values; a luma block of a 1080p key frame 2.5k cycles instead of
+ * 2.9k, a 4x4 of the depth search 2.2k instead of 3.0 - 4.4k. */
+DEVI void wave_predict8(uint8_t *px, int S, int sx, int sy, int lw, int lh, int mode, int delta, int hl, int ha, int har,
+                        int hbl, int maxX, int maxY, int edgeFilter, int filterType, int *eA, int *eL) {
+  S = d_uni(S);
+  sx = d_uni(sx);
+  sy = d_uni(sy);
+  lw = d_uni(lw);
+  lh = d_uni(lh);
+  mode = d_uni(mode);
+  delta = d_uni(delta);
+  hl = d_uni(hl);
+  ha = d_uni(ha);
+  har = d_uni(har);
+  hbl = d_uni(hbl);
+  const int lane = d_local(threadIdx.x & 63), half = lane >> 5, k = (lane & 31) - 1, w = 1 << lw, h = 1 << lh;
+  const lds_u8 *lpx = (const lds_u8 *)px;
+  /* 7.11.2 steps 1-3: the neighbouring samples */
+  int e;
+  if (ha || hl) {
+    const int aLim = d_min(maxX, sx + (har ? 2 * w : w) - 1), lLim = d_min(maxY, sy + (hbl ? 2 * h : h) - 1);
+    int X = half ? sx - 1 : d_min(aLim, sx + k), Y = half ? d_min(lLim, sy + k) : sy - 1;
+    if (!(ha && hl)) {
+      const bool mine = k >= 0 && (half ? hl : ha);
+      if (!mine) {
+        X = ha ? sx : sx - 1;
+        Y = ha ? sy - 1 : sy;
+      }
+    }
+    e = lpx[Y * S + X];
+  } else {
+    e = k < 0 ? 128 : half ? 129 : 127;
+  }
+  IntraMode im;
+  intra_mode_setup(im, mode, delta, lw, lh);
+  im.pAngle = d_uni(im.pAngle);
+  im.dx = d_uni(im.dx);
+  im.dy = d_uni(im.dy);
+  im.corner = __builtin_amdgcn_readlane(e, 0);
+  im.dcv = 0;
+  if (mode == DC_PRED) {
+    const bool use = k >= 0 && (half ? hl && k < h : ha && k < w);
+    const int sum = wave_sum_dpp(use ? e : 0);
+    im.dcv = (ha && hl) ? (lw == lh ? (sum + w) >> (lw + 1) : (sum + ((w + h) >> 1)) / (w + h))
+             : hl       ? (sum + (h >> 1)) >> lh
+             : ha       ? (sum + (w >> 1)) >> lw
+                        : 128;
+  } else {
+    int up = 0; /* this half's edge is upsampled */
+    int e2 = 0;
+    if (mode >= V_PRED && mode <= D67_PRED && edgeFilter) {
+      const int pa = im.pAngle;
+      if (pa != 90 && pa != 180) {
+        const int sA = ha ? edge_strength(w, h, filterType, pa - 90) : 0;
+        const int sL = hl ? edge_strength(w, h, filterType, pa - 180) : 0;
+        if (d_uni(sA | sL)) {
+          const int st = half ? sL : sA;
+          const int sz = half ? d_min(h, maxY - sy + 1) + (pa > 180 ? w : 0) + 1 : d_min(w, maxX - sx + 1) + (pa < 90 ? h : 0) + 1;
+          const int i = k + 1, base = lane & 32;
+          const int c0 = __shfl(e, base + d_clip(0, sz - 1, i - 2)), c1 = __shfl(e, base + d_clip(0, sz - 1, i - 1));
+          const int c3 = __shfl(e, base + d_clip(0, sz - 1, i + 1)), c4 = __shfl(e, base + d_clip(0, sz - 1, i + 2));
+          /* the kernels of 7.11.2.12: {0 4 8 4 0}, {0 5 6 5 0}, {2 4 4 4 2} */
+          const int k1 = st == 2 ? 5 : 4, k2 = st == 1 ? 8 : st == 2 ? 6 : 4;
+          int s = k2 * e + k1 * (c1 + c3);
+          if (st == 3) s += 2 * (c0 + c4);
+          if (st > 0 && i >= 1 && i < sz) e = (s + 8) >> 4;
+        }
+      }
+      im.upA = d_uni(use_upsample(w, h, filterType, pa - 90));
+      im.upL = d_uni(use_upsample(w, h, filterType, pa - 180));
+      if (im.upA || im.upL) {
+        up = half ? im.upL : im.upA;
+        const int n = half ? h + (pa > 180 ? w : 0) : w + (pa < 90 ? h : 0), base = (lane & 32) + 1;
+        const int m2 = __shfl(e, base + d_max(-1, k - 2)), m1 = __shfl(e, base + d_max(-1, k - 1));
+        const int p1 = __shfl(e, base + d_min(n - 1, k + 1));
+        e2 = d_clip1(d_round2(9 * (m1 + e) - m2 - p1, 4));
+        /* lanes past the upsampled samples write nothing */
+        if (up && k >= n) up = 2;
+      }
+    }
+    lds_i32 *E = half ? lds(eL) + EDGE_NEG : lds(eA) + EDGE_NEG;
+    if (up == 0) {
+      if (k < w + h) E[k] = e;
+    } else if (up == 1) {
+      E[2 * k] = e;                  /* k = -1: the corner moves to -2 */
+      if (k >= 0) E[2 * k - 1] = e2;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+  if (lane < w * h) {
+    const int i = lane >> lw, j = lane & (w - 1);
+    px[(sy + i) * S + sx + j] = (uint8_t)intra_px(im, eA + EDGE_NEG, eL + EDGE_NEG, i, j);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+/* The prediction of a transform block by one wave. */
+DEVI void wave_predict(uint8_t *px, int S, int sx, int sy, int lw, int lh, int mode, int delta, int hl, int ha, int har,
+                       int hbl, int maxX, int maxY, int edgeFilter, int filterType, SiWave &W) {
+  if (d_uni(lw) <= 3 && d_uni(lh) <= 3)
+    wave_predict8(px, S, sx, sy, lw, lh, mode, delta, hl, ha, har, hbl, maxX, maxY, edgeFilter, filterType, W.eA, W.eL);
+  else
+    intra_tx_predict(wave_ctx(), px, S, sx, sy, lw, lh, mode, delta, hl, ha, har, hbl, maxX, maxY, edgeFilter,
+                     filterType, W.eA, W.eL, W.ecp);
 }
 
 /* CfL (7.11.5) over the DC prediction in px: the alpha with the smallest
@@ -672,12 +924,12 @@ DEVI void si_predict(const Mav1FrameParams &fp, Mav1BlockInfo &b, int plane, SiW
   const int availU = mr > 0, availL = mc > tile_start(fp, mc);
   const int uvMode = d_uni(b.uv_mode);
   const int isCfl = plane > 0 && uvMode == UV_CFL_PRED;
-  intra_tx_predict(c, g.px, g.S, g.sx, g.sy, g.lw, g.lh, d_uni(plane == 0 ? b.y_mode : (isCfl ? DC_PRED : uvMode)),
+  wave_predict(g.px, g.S, g.sx, g.sy, g.lw, g.lh, d_uni(plane == 0 ? b.y_mode : (isCfl ? DC_PRED : uvMode)),
                    d_uni(plane == 0 ? b.angle_y : b.angle_uv), availL, availU,
                    d_uni(har >= 0 ? har : gL.bd[BDI(plane, (sbr >> sub) - 1, (sbc >> sub) + stepX)]),
                    d_uni(hbl >= 0 ? hbl : gL.bd[BDI(plane, (sbr >> sub) + stepY, (sbc >> sub) - 1)]),
                    ((fp.mi_cols * 4) >> sub) - 1, ((fp.mi_rows * 4) >> sub) - 1, fp.enable_intra_edge_filter,
-                   d_uni((b.interp_filter >> (plane == 0 ? 4 : 5)) & 1), W.eA, W.eL, W.ecp);
+                   d_uni((b.interp_filter >> (plane == 0 ? 4 : 5)) & 1), W);
   if (!isCfl) return;
   /* CfL (7.11.5) over the DC prediction: the luma average of each sample,
    * then one alpha per lane */
@@ -753,15 +1005,19 @@ DEVI void si_code_chroma(const Mav1FrameParams &fp, Mav1BlockInfo &b, int plane,
   const int set = d_uni(get_tx_set(g.txSz, 0, fp.reduced_tx_set));
   int t = d_uni(Mode_To_Txfm[d_uni(b.uv_mode)]);
   if (d_uni(Tx_Size_Sqr_Up[g.txSz]) > TX_32X32 || !d_uni(in_set(set, t, 0))) t = DCT_DCT;
-  long long cost;
-  const int eob = tx_eval<true>(c, fp, g.spx, g.S, g.px, g.S, g.sx, g.sy, g.txSz, plane, t, true, T.resid, SRS, T.tmp, T.coef,
-                          T.q, T.dq, SQS, mats, &cost);
-  const int type = eob > 0 ? t : DCT_DCT;
   const int tw = d_min(32, 1 << g.lw), th = d_min(32, 1 << g.lh);
   int32_t *co = coefs + d_uni(b.coef_off[plane]);
+  int eob;
+  if (g.txSz == TX_4X4) {
+    eob = wave_tx4(fp, plane, g.spx, g.S, g.px, g.S, g.sx, g.sy, t, T.q);
+  } else {
+    long long cost;
+    eob = tx_eval<true>(c, fp, g.spx, g.S, g.px, g.S, g.sx, g.sy, g.txSz, plane, t, true, T.resid, SRS, T.tmp, T.coef,
+                        T.q, T.dq, SQS, mats, &cost);
+    if (eob > 0)
+      wave_recon_any(c, T.q, T.resid, g.txSz, t, fp.dc_q[plane], fp.ac_q[plane], g.px, g.S, g.sx, g.sy);
+  }
   for (int k = c.tid; k < tw * th; k += 64) co[k] = T.q[k];
-  if (eob > 0)
-    tx_recon_small(c, T.q, T.resid, SRS, g.txSz, type, fp.dc_q[plane], fp.ac_q[plane], g.px, g.S, g.sx, g.sy);
   if (c.tid == 0) b.eob[plane] = eob > 0;
 }
 
@@ -941,7 +1197,8 @@ DEVI void lvl_publish(unsigned long long *m, int i) {
  * deepest depth's wave. Coding each transform block by the whole workgroup
  * took about 30k cycles with its five barriers (11.3M per superblock); two
  * waves per block and one block per team let independent blocks, depths and
- * chroma run side by side: five full-RD frames of 1280x720 289 -> 80 ms. */
+ * chroma run side by side: five full-RD frames of 1280x720 took 289 ms, with
+ * this split 80 ms, with the waves' transforms in registers 62 ms. */
 
 /* The private pixel copy addressed by plane position, for the block at luma
  * (x0, y0). */
@@ -971,7 +1228,6 @@ DEVI RdRes rd_depth(const Mav1FrameParams &fp, const Mav1BlockInfo &b, int depth
    * then the left column to twice the height (inside the tile; rows below
    * it are never read) */
   {
-    typedef __attribute__((address_space(3))) uint32_t lds_u32;
     const int nc = 2 * n4w + 1, w = n4w * 4, h = n4h * 4, cx = lane & 15, bottom = (mr | 15) * 4 + 3;
     (void)w;
     if (cx < nc)
@@ -1004,8 +1260,13 @@ DEVI RdRes rd_depth(const Mav1FrameParams &fp, const Mav1BlockInfo &b, int depth
        * transform row before; below-left: from the column left of the block */
       const int har = ty == 0 ? (av >> (tx + stepX)) & 1 : tx + stepX < n4w;
       const int hbl = tx == 0 ? (av >> (8 + ty + stepY)) & 1 : 0;
-      intra_tx_predict(c, px, RD_PS, sx, sy, lw, lh, mode, delta, availL || tx > 0, availU || ty > 0, har, hbl, maxX - 1,
-                       maxY - 1, fp.enable_intra_edge_filter, ft, P.eA, P.eL, P.ecp);
+      const int hl = availL || tx > 0, ha = availU || ty > 0;
+      if constexpr (DEEP)
+        wave_predict8(px, RD_PS, sx, sy, 2, 2, mode, delta, hl, ha, har, hbl, maxX - 1, maxY - 1,
+                      fp.enable_intra_edge_filter, ft, P.eA, P.eL);
+      else
+        wave_predict(px, RD_PS, sx, sy, lw, lh, mode, delta, hl, ha, har, hbl, maxX - 1, maxY - 1,
+                     fp.enable_intra_edge_filter, ft, P);
       int32_t *lv = lev + R.n * area;
       int t = DCT_DCT, eob = 0;
       long long cost;
@@ -1029,7 +1290,7 @@ DEVI RdRes rd_depth(const Mav1FrameParams &fp, const Mav1BlockInfo &b, int depth
           }
         }
         if (eob > 0)
-          tx_recon_small(c, lv, W->resid, SRS, txSz, t, fp.dc_q[0], fp.ac_q[0], px, RD_PS, sx, sy);
+          wave_recon_any(c, lv, W->resid, txSz, t, fp.dc_q[0], fp.ac_q[0], px, RD_PS, sx, sy);
       }
       R.cost += cost;
       if (R.n < 16) R.types |= (unsigned long long)t << (4 * R.n);
@@ -1079,7 +1340,6 @@ DEVI void rd_join(const Mav1FrameParams &fp, int i, int team, int slot, const Rd
   const int bs = d_uni(b.bsize), mr = d_uni(b.mi_row), mc = d_uni(b.mi_col), x0 = mc * 4, y0 = mr * 4;
   const int lw4 = d_uni(Num_4x4_Blocks_Wide[bs]) == 4 ? 2 : 1, n4h = d_uni(Num_4x4_Blocks_High[bs]);
   {
-    typedef __attribute__((address_space(3))) uint32_t lds_u32;
     int TS;
     uint8_t *tile = tile_ptr(0, 0, mr, mc, TS);
     const uint8_t *px = rd_pix(pix, x0, y0);
@@ -1192,7 +1452,7 @@ DEVI void lvl_dataflow(const Mav1FrameParams &fp, int32_t *__restrict__ coefs, c
          * its pixels; then the levels out and the block's transform fields
          * (lvl_luma_out's work, in that order) */
         if (eob > 0)
-          tx_recon_small(c, W.q, W.resid, SRS, g.txSz, DCT_DCT, fp.dc_q[0], fp.ac_q[0], g.px, g.S, g.sx, g.sy);
+          wave_recon_any(c, W.q, W.resid, g.txSz, DCT_DCT, fp.dc_q[0], fp.ac_q[0], g.px, g.S, g.sx, g.sy);
         lvl_publish(&L.ldm, i);
         const int tw = d_min(32, 1 << g.lw), th = d_min(32, 1 << g.lh);
         int32_t *co = coefs + d_uni(b.coef_off[0]);
