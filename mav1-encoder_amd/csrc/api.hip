@@ -64,7 +64,6 @@ struct mav1hip_ctx {
   Mav1LrUnit *d_lrunits;
   int8_t *d_choice;
   void *d_lrstats;
-  void *d_lrchain;
   int *d_lrtype, *d_lrreruns;
   uint8_t *d_decgrid;
   int *d_rwork;
@@ -72,7 +71,6 @@ struct mav1hip_ctx {
   int num_cu;
   size_t decgrid_bytes;
   int lr_units;
-  int lr_gen; /* generation of the last restoration fit launch */
   long entry_bytes;
   size_t planes_bytes;
   /* frames the stages read (own buffers or pool frames) */
@@ -293,10 +291,6 @@ static mav1hip_ctx *create_ctx(const Mav1HipConfig *cfg, hipStream_t extMain, hi
     }
     rc |= dmalloc(c, (void **)&c->d_lrunits, sizeof(Mav1LrUnit) * (size_t)c->lr_units);
     rc |= dmalloc(c, &c->d_lrstats, lr_stat_bytes() * (size_t)c->lr_units);
-    /* zeroed once: the fit's generation numbers start at 1 */
-    if (rc == MAV1HIP_OK && hipMemset(c->d_lrstats, 0, lr_stat_bytes() * (size_t)c->lr_units) != hipSuccess)
-      rc = fail(c, MAV1HIP_EDEVICE, "hipMemset of the restoration statistics failed");
-    rc |= dmalloc(c, &c->d_lrchain, lr_chain_bytes());
     rc |= dmalloc(c, (void **)&c->d_lrtype, sizeof(int) * 3);
     rc |= dmalloc(c, (void **)&c->d_lrreruns, sizeof(int) * 3);
   }
@@ -379,7 +373,6 @@ void mav1hip_destroy(mav1hip_ctx *c) {
   (void)hipFree(c->d_iwork);
   (void)hipFree(c->d_lrunits);
   (void)hipFree(c->d_lrstats);
-  (void)hipFree(c->d_lrchain);
   (void)hipFree(c->d_lrtype);
   (void)hipFree(c->d_lrreruns);
   (void)hipFree(c->d_pool);
@@ -672,31 +665,14 @@ int mav1hip_launch_lr_select(mav1hip_ctx *c, int32_t lr_test) {
   if (!c || !c->fp_set) return fail(c, MAV1HIP_EINVAL, "lr select: no frame parameters set");
   int rc = check_lr_params(c, c->fp);
   if (rc) return rc;
-  c->lr_gen = c->lr_gen % 0x7ffffffe + 1;
   if ((rc = timed(c, "lr_fit", [&] {
-         return launch_lr_fit(c->stream, c->fp, c->b_src, c->d_rec, c->d_dbk, c->d_lrstats, c->d_lrchain, c->lr_units,
-                              c->lr_gen);
+         return launch_lr_fit(c->stream, c->fp, c->b_src, c->d_rec, c->d_dbk, c->d_lrstats, c->lr_units);
        })))
     return rc;
-  /* the fit launch refines under the default reference; then up to
-   * LR_ROUNDS - 1 chain launches that stop at a reference change, each
-   * followed by the refinement of the remaining units under the new
-   * reference; the last chain launch refines any further mismatching unit
-   * itself */
-  const int LR_ROUNDS = 3;
-  for (int r = 0; r < LR_ROUNDS; r++) {
-    if (r > 0 && (rc = timed(c, "lr_path", [&] {
-                    return launch_lr_path(c->stream, c->fp, c->b_src, c->d_rec, c->d_dbk, c->d_lrstats, c->d_lrchain,
-                                          c->lr_units);
-                  })))
-      return rc;
-    if ((rc = timed(c, "lr_chain", [&] {
-           return launch_lr_chain(c->stream, c->fp, c->b_src, c->d_rec, c->d_dbk, c->d_lrstats, c->d_lrunits,
-                                  c->d_lrtype, lr_test != 0, c->d_lrreruns, c->d_lrchain, r < LR_ROUNDS - 1);
-         })))
-      return rc;
-  }
-  return MAV1HIP_OK;
+  return timed(c, "lr_chain", [&] {
+    return launch_lr_chain(c->stream, c->fp, c->b_src, c->d_rec, c->d_dbk, c->d_lrstats, c->d_lrunits, c->d_lrtype,
+                           lr_test != 0, c->d_lrreruns);
+  });
 }
 
 int mav1hip_lr_select(mav1hip_ctx *c, const Mav1FrameParams *fp, const uint8_t *src, const uint8_t *cdef,
@@ -1029,7 +1005,7 @@ int ctx_clear_choice(mav1hip_ctx *c) {
   HIPCHK(c, hipMemsetAsync(c->d_choice, 0, (size_t)c->num_sbs, c->stream));
   return MAV1HIP_OK;
 }
-int ctx_batch_frame(mav1hip_ctx *c, BatchFrame *bf, int new_lr_gen) {
+int ctx_batch_frame(mav1hip_ctx *c, BatchFrame *bf) {
   if (!c || !bf || !c->fp_set) return MAV1HIP_EINVAL;
   memset(bf, 0, sizeof *bf);
   bf->fp = c->fp;
@@ -1060,13 +1036,10 @@ int ctx_batch_frame(mav1hip_ctx *c, BatchFrame *bf, int new_lr_gen) {
   bf->choice = c->d_choice;
   bf->lrunits = c->d_lrunits;
   bf->lrstats = c->d_lrstats;
-  bf->lrchain = c->d_lrchain;
   bf->lrtype = c->d_lrtype;
   bf->lrreruns = c->d_lrreruns;
   bf->frame_bytes = (long long)c->frame_bytes;
   bf->lr_units = c->lr_units;
-  if (new_lr_gen) c->lr_gen = c->lr_gen % 0x7ffffffe + 1;
-  bf->lr_gen = c->lr_gen;
   c->me_pending = 0;
   return MAV1HIP_OK;
 }

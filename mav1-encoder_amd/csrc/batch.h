@@ -43,10 +43,10 @@ struct BatchFrame {
   int *dirvar;
   int8_t *choice;
   Mav1LrUnit *lrunits;
-  void *lrstats, *lrchain;
+  void *lrstats;
   int *lrtype, *lrreruns;
   long long frame_bytes;
-  int lr_units, lr_gen;
+  int lr_units;
   /* the deepest analysis level per superblock the pruner allows (NULL: no
    * pruning) */
   int8_t *prune;
@@ -125,8 +125,7 @@ hipError_t launch_cdef_select_b(hipStream_t st, const BatchFrame *T, const Batch
 hipError_t launch_lr_apply_b(hipStream_t st, const BatchFrame *T, const BatchFrame *H, int n);
 hipError_t launch_decision_grid_b(hipStream_t st, const BatchFrame *T, const BatchFrame *H, int n);
 hipError_t launch_lr_fit_b(hipStream_t st, const BatchFrame *T, const BatchFrame *H, int n);
-hipError_t launch_lr_path_b(hipStream_t st, const BatchFrame *T, const BatchFrame *H, int n);
-hipError_t launch_lr_chain_b(hipStream_t st, const BatchFrame *T, const BatchFrame *H, int n, int lrTest, int stop);
+hipError_t launch_lr_chain_b(hipStream_t st, const BatchFrame *T, int n, int lrTest);
 /* Frame copies and clears of the driver: which 0 = reconstruction into the
  * deblocked copy, 1 = reconstruction into the restoration output, 2 = the
  * CDEF choices cleared. */

@@ -67,25 +67,17 @@ hipError_t launch_decision_grid(hipStream_t st, const Mav1FrameParams &fp, const
                                 const Mav1SbInfo *sbs, uint8_t *grid);
 
 /* lrsearch.hip */
-/* Upper bounds of lr_stat_bytes() and lr_chain_bytes() (the static scratch
- * of mav1hip_lr_select_static is laid out with them). */
+/* Upper bound of lr_stat_bytes() (the static scratch of
+ * mav1hip_lr_select_static is laid out with it). */
 #define LR_STAT_MAX_BYTES 384
-#define LR_CHAIN_MAX_BYTES 192
 size_t lr_stat_bytes();
-size_t lr_chain_bytes();
-/* The fit of every unit with its refinement under the default reference,
- * and the chain state reset. gen: a number that differs from the previous
- * launch's on the same statistics buffer (the buffer starts zeroed). */
+/* The fit of every unit with its refinement under the default reference. */
 hipError_t launch_lr_fit(hipStream_t st, const Mav1FrameParams &fp, const uint8_t *src, const uint8_t *cdef,
-                         const uint8_t *dbk, void *stats, void *chain, int nunits, int gen);
-/* Refinement of the units from each plane's chain restart point on. */
-hipError_t launch_lr_path(hipStream_t st, const Mav1FrameParams &fp, const uint8_t *src, const uint8_t *cdef,
-                          const uint8_t *dbk, void *stats, const void *chain, int nunits);
-/* The unit chains; stop: end at the first reference mismatch instead of
- * refining the unit again. */
+                         const uint8_t *dbk, void *stats, int nunits);
+/* The unit chains. */
 hipError_t launch_lr_chain(hipStream_t st, const Mav1FrameParams &fp, const uint8_t *src, const uint8_t *cdef,
                            const uint8_t *dbk, const void *stats, Mav1LrUnit *units, int *lrType, int lrTest,
-                           int *reruns, void *chain, int stop);
+                           int *reruns);
 
 /* api.hip: library-internal access to a context for the sequence driver */
 /* A context on two streams the caller keeps (neither created nor destroyed
@@ -107,9 +99,8 @@ int ctx_store(mav1hip_ctx *c, uint8_t *dst, int buf);
 int ctx_rec_to_lrout(mav1hip_ctx *c);
 int ctx_clear_choice(mav1hip_ctx *c);
 /* The context's frame as a batch table entry: its parameters (set by
- * mav1hip_set_params), bound inputs and buffers. new_lr_gen: take the next
- * restoration-fit generation, as a restoration search of this context does. */
-int ctx_batch_frame(mav1hip_ctx *c, BatchFrame *bf, int new_lr_gen);
+ * mav1hip_set_params), bound inputs and buffers. */
+int ctx_batch_frame(mav1hip_ctx *c, BatchFrame *bf);
 /* workgroups of the persistent inter and intra phases */
 int ctx_num_cu(const mav1hip_ctx *c);
 

@@ -870,7 +870,7 @@ int round_early(mav1hip_batch *b, Round &R) {
   BatchFrame *T = b->d_tab + (size_t)R.tab * kMaxBatch, *H = b->h_tab + (size_t)R.tab * kMaxBatch;
   const bool prune = b->pruner[e] && b->prune_tau > 0.f;
   for (int k = 0, off = 0; k < n; k++) {
-    if (ctx_batch_frame(R.seqs[k]->eng[e].ctx, &H[k], R.frames[k].plan.restoration))
+    if (ctx_batch_frame(R.seqs[k]->eng[e].ctx, &H[k]))
       return bfail(b, MAV1HIP_EINVAL, "batch: frame %d has no parameters", k);
     H[k].prune = prune ? b->d_prune[e] + off : nullptr;
     off += H[k].fp.sb_cols * H[k].fp.sb_rows;
@@ -958,14 +958,8 @@ int round_late(mav1hip_batch *b, Round &R) {
   else if (cdefOff)
     LCHK(b, "cdef choice clear", launch_frame_op_b(st, T, H, n, 2));
   if (pl.restoration) {
-    /* the fit, then chain launches with the refinements between them, as
-     * the single-frame restoration search */
-    const int LR_ROUNDS = 3;
     LCHK(b, "lr_fit", launch_lr_fit_b(st, T, H, n));
-    for (int r = 0; r < LR_ROUNDS; r++) {
-      if (r > 0) LCHK(b, "lr_path", launch_lr_path_b(st, T, H, n));
-      LCHK(b, "lr_chain", launch_lr_chain_b(st, T, H, n, b->lr_test != 0, r < LR_ROUNDS - 1));
-    }
+    LCHK(b, "lr_chain", launch_lr_chain_b(st, T, n, b->lr_test != 0));
     LCHK(b, "restoration copy", launch_frame_op_b(st, T, H, n, 1));
     LCHK(b, "lr_apply", launch_lr_apply_b(st, T, H, n));
   }
