@@ -7,15 +7,14 @@
  * non-trivial horizontal phases are filtered once per row into LDS, and
  * each thread produces 4 adjacent pixels of all 16 phase planes.
  *
- * Node search: one wave64 per (node, reference). Full-pel candidates are
- * spread over the lanes (lane k evaluates candidates k, k + 64, ...), each
- * scored against the source block and the +-range search window staged in
- * LDS (edge clamping applied while staging, which reproduces the
- * per-coordinate clamping of the serial search); the winner is the
- * lexicographic minimum of (cost, candidate index) over the wave, i.e. the
- * serial loop's first minimum. Sub-pel steps spread the 4x4 units of one
- * candidate over the lanes and sum with a wave reduction; candidates are
- * compared in ring order with a strict <, as the serial refinement does.
+ * Node search: one workgroup per (node, reference). A few lanes share a
+ * full-pel candidate, scored against the source block and the +-range search
+ * window staged in LDS (edge clamping applied while staging, which
+ * reproduces the per-coordinate clamping of the serial search); the winner is
+ * the lexicographic minimum of (cost, candidate index), i.e. the serial
+ * loop's first minimum. Sub-pel steps spread the 4x4 units of all of a ring's
+ * candidates over the lanes; candidates are compared in ring order with a
+ * strict <, as the serial refinement does.
  * Levels depend on their parent level and run as separate launches.
  */
 #include "dev_common.h"
@@ -137,7 +136,18 @@ hipError_t launch_dec_build(hipStream_t st, const Mav1FrameParams &fp, const uin
 /* ------------------------------------------------------------------------ */
 /* Node search                                                               */
 /* ------------------------------------------------------------------------ */
-#define WIN_R 4 /* largest full-pel radius served from the LDS window */
+/* Threads of a node's workgroup and, in the full-pel stages, the lanes that
+ * share a candidate (each takes every ME_G-th row): many for the few large
+ * nodes, whose 50 to 290 candidates of up to 4096 samples are a node's
+ * latency; one wave for the 16x16 and 8x8 nodes, which fill the chip. */
+template <int LEVEL>
+constexpr int ME_NT = LEVEL == 0 ? 512 : LEVEL == 1 ? 256 : 64;
+template <int LEVEL>
+constexpr int ME_G = LEVEL <= 1 ? 8 : 2;
+/* Largest full-pel radius served from the LDS window. */
+template <int LEVEL>
+constexpr int ME_WIN = LEVEL == 0 ? 32 : 4;
+#define ME_DEC_R 8 /* largest radius of the decimated window (full-pel radius 32) */
 
 struct NodeState {
   int x, y, cy, cx, range, step, nstage, pr, pc, copy, valid;
@@ -159,152 +169,155 @@ DEVI int me_bits(int dy, int dx) {
   return 2 + 2 * d_floorlog2((unsigned)(d_abs(dy) * 8 + 1)) + 2 * d_floorlog2((unsigned)(d_abs(dx) * 8 + 1));
 }
 
-template <int BW>
-DEVI int sad_lds(const uint8_t *srcL, const uint8_t *win, int WW, int oy, int ox, int rs) {
-  int s = 0;
-  for (int i = 0; i < BW; i += rs) {
-    const uint8_t *a = srcL + i * BW, *b = win + (i + oy) * WW + ox;
-#pragma unroll 8
-    for (int j = 0; j < BW; j++) s += d_abs((int)a[j] - (int)b[j]);
+typedef __attribute__((address_space(3))) const uint32_t lds_cu32;
+/* Byte `at` on of an LDS array of words, as words. */
+struct LdsBytes {
+  const lds_cu32 *p;
+  uint32_t w;
+  int s;
+  DEVI LdsBytes(const uint8_t *base, int at) {
+    p = (const lds_cu32 *)(base + (at & ~3));
+    s = at & 3;
+    w = *p++;
   }
-  return s * rs;
+  DEVI uint32_t next() {
+    const uint32_t n = *p++, v = __builtin_amdgcn_alignbyte(n, w, s);
+    w = n;
+    return v;
+  }
+};
+/* SAD of rows first, + stride, .. of an N x N block at srcL (row stride N)
+ * against the window (row stride WS) from (oy, ox) on. */
+template <int N, int WS>
+DEVI int sad_rows(const uint8_t *srcL, const uint8_t *win, int oy, int ox, int first, int stride) {
+  uint32_t s = 0;
+  for (int i = first; i < N; i += stride) {
+    const lds_cu32 *a = (const lds_cu32 *)(srcL + i * N);
+    LdsBytes b(win, (i + oy) * WS + ox);
+#pragma unroll
+    for (int j = 0; j < N / 4; j++) s = __builtin_amdgcn_sad_u8(a[j], b.next(), s);
+  }
+  return (int)s;
 }
-
+/* The same against the frame (coordinates clamped), for radii past the window. */
 template <int BW>
-DEVI int sad_global(const Mav1FrameParams &fp, const uint8_t *srcL, const uint8_t *refY, int x, int y, int dy, int dx,
-                    int rs) {
+DEVI int sad_rows_global(const Mav1FrameParams &fp, const uint8_t *srcL, const uint8_t *refY, int x, int y, int dy,
+                         int dx, int first, int stride) {
   int s = 0, S = fp.stride[0];
-  for (int i = 0; i < BW; i += rs) {
+  for (int i = first; i < BW; i += stride) {
     const uint8_t *b = refY + d_clip(0, fp.frame_h - 1, y + i + dy) * S;
     for (int j = 0; j < BW; j++) s += d_abs((int)srcL[i * BW + j] - (int)b[d_clip(0, fp.frame_w - 1, x + j + dx)]);
   }
-  return s * rs;
+  return s;
 }
-
 template <int BW>
-DEVI int sad_dec(const Mav1FrameParams &fp, const uint8_t *ds, const uint8_t *dr, int x, int y, int dy, int dx) {
+DEVI int sad_rows_dec_global(const Mav1FrameParams &fp, const uint8_t *ds, const uint8_t *dr, int x, int y, int dy,
+                             int dx, int first, int stride) {
   const int W = (fp.frame_w + 3) >> 2, H = (fp.frame_h + 3) >> 2, n = BW >> 2;
   const int x0 = x >> 2, y0 = y >> 2, oy = dy >> 2, ox = dx >> 2;
   int s = 0;
-  for (int i = 0; i < n; i++) {
+  for (int i = first; i < n; i += stride) {
     const uint8_t *a = ds + d_min(y0 + i, H - 1) * W, *b = dr + d_clip(0, H - 1, y0 + i + oy) * W;
     for (int j = 0; j < n; j++) s += d_abs((int)a[d_min(x0 + j, W - 1)] - (int)b[d_clip(0, W - 1, x0 + j + ox)]);
   }
-  return s * 16;
+  return s;
+}
+/* Sum over the G lanes that share a candidate (in every one of them). */
+template <int G>
+DEVI int me_group_sum(int v) {
+  v += dpp_t<DPP_QX1>(v);
+  if constexpr (G == 8) {
+    v += dpp_t<DPP_QX2>(v);
+    v += dpp_t<DPP_HMIRROR>(v);
+  }
+  return v;
 }
 
-/* Sub-pel cost at an even 1/8-pel vector from the quarter-pel planes: the
- * SATD of every st-th 4x4 unit (raster order), summed over the wave. */
-template <int BW>
-DEVI int subpel_cost_hp(const Mav1FrameParams &fp, const uint8_t *srcL, const uint8_t *planes, int x, int y, int mvr,
-                        int mvc, int st, int lane) {
-  constexpr int NR = BW / 4, NU = NR * NR;
-  const int W = fp.frame_w, H = fp.frame_h;
-  const uint8_t *pl = planes + (size_t)(((mvr >> 1) & 3) * 4 + ((mvc >> 1) & 3)) * W * H;
-  int s = 0;
-  for (int u = lane * st; u < NU; u += 64 * st) {
-    int ucol = u % NR, urow = u / NR;
-    int iy = y + urow * 4 + (mvr >> 3), ix = x + ucol * 4 + (mvc >> 3);
-    int d[16];
+/* The normative EIGHTTAP prediction (7.11.3) of a 4x4 unit at an even
+ * 1/8-pel vector, from the staged window: (wy, wx) the window position of the
+ * unit's first sample, phases fy, fx in quarter samples. d: source minus
+ * prediction. The horizontal taps are signed bytes times (sample - 128) on
+ * the dot products (the whole-sample phase's 128 as 2 * 64), the vertical
+ * ones pairs of 16 bits. */
+struct MeTaps {
+  uint32_t h[4][2], v[4][4];
+};
+DEVI void me_taps(MeTaps &T, int tid) {
+  if (tid < 4) {
+    const int16_t *k = SUBPEL_FILTER(EIGHTTAP, 4 * tid);
+    uint32_t w[2] = {0, 0};
+    for (int t = 0; t < 8; t++) {
+      w[t >> 2] |= (uint32_t)((tid ? k[t] : k[t] / 2) & 255) << (8 * (t & 3));
+      if (!(t & 1)) T.v[tid][t >> 1] = (uint32_t)(k[t] & 0xFFFF) | (uint32_t)(k[t + 1] & 0xFFFF) << 16;
+    }
+    T.h[tid][0] = w[0];
+    T.h[tid][1] = w[1];
+  }
+}
+template <int WS>
+DEVI void me_pred_diff(const MeTaps &T, const uint8_t *win, int wy, int wx, int fy, int fx, const uint32_t src[4],
+                       int d[16]) {
+  typedef short s2 __attribute__((ext_vector_type(2)));
+  union P {
+    uint32_t u;
+    s2 v;
+  };
+  const int t0 = (int)T.h[fx][0], t1 = (int)T.h[fx][1], sh = fx ? 0 : 1;
+  int m[4][11];
+#pragma unroll
+  for (int r = 0; r < 11; r++) {
+    LdsBytes b(win, (wy - 3 + r) * WS + wx - 3);
+    const uint32_t n0 = b.next() ^ 0x80808080u, n1 = b.next() ^ 0x80808080u, n2 = b.next() ^ 0x80808080u;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const int lo = (int)__builtin_amdgcn_alignbyte(n1, n0, j), hi = (int)__builtin_amdgcn_alignbyte(n2, n1, j);
+      const int a = __builtin_amdgcn_sdot4(hi, t1, __builtin_amdgcn_sdot4(lo, t0, 0, false), false);
+      m[j][r] = ((a << sh) + 16384 + 4) >> 3;
+    }
+  }
+  P v[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) v[i].u = T.v[fy][i];
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    P p[10];
+#pragma unroll
+    for (int r = 0; r < 10; r++) p[r].u = ((uint32_t)m[j][r] & 0xFFFF) | (uint32_t)m[j][r + 1] << 16;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      const uint8_t *prow = pl + (size_t)d_clip(0, H - 1, iy + i) * W;
-      const uint8_t *srow = srcL + (urow * 4 + i) * BW + ucol * 4;
+      int a = 1 << 10;
 #pragma unroll
-      for (int j = 0; j < 4; j++) d[4 * i + j] = (int)srow[j] - (int)prow[d_clip(0, W - 1, ix + j)];
+      for (int t = 0; t < 4; t++) a = __builtin_amdgcn_sdot2(p[i + 2 * t].v, v[t].v, a, false);
+      d[4 * i + j] = (int)((src[i] >> (8 * j)) & 255) - d_clip1(a >> 11);
     }
-    s += satd4x4_arr(d);
   }
-  return wave_sum(s) * st;
 }
 
-/* Sub-pel costs of up to 9 candidates at once from the quarter-pel planes:
- * the lanes take (candidate, 4x4 unit) pairs, and each candidate's cost is
- * the same sum as subpel_cost_hp's (every st-th unit, times st), added up
- * in LDS. Integer sums, so the order does not matter. */
-template <int BW>
-DEVI void subpel_costs_hp(const Mav1FrameParams &fp, const uint8_t *srcL, const uint8_t *planes, int x, int y,
-                          const int *cr, const int *cc, int ncand, int st, int lane, int *cost) {
-  constexpr int NR = BW / 4, NU = NR * NR;
-  const int W = fp.frame_w, H = fp.frame_h, nue = NU / st;
-  if (lane < ncand) cost[lane] = 0;
-  __syncthreads();
-  for (int p = lane; p < ncand * nue; p += 64) {
-    const int c = p / nue, u = (p - c * nue) * st;
-    const int mvr = cr[c], mvc = cc[c];
-    const uint8_t *pl = planes + (size_t)(((mvr >> 1) & 3) * 4 + ((mvc >> 1) & 3)) * W * H;
-    const int ucol = u % NR, urow = u / NR;
-    const int iy = y + urow * 4 + (mvr >> 3), ix = x + ucol * 4 + (mvc >> 3);
-    int d[16];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const uint8_t *prow = pl + (size_t)d_clip(0, H - 1, iy + i) * W;
-      const uint8_t *srow = srcL + (urow * 4 + i) * BW + ucol * 4;
-#pragma unroll
-      for (int j = 0; j < 4; j++) d[4 * i + j] = (int)srow[j] - (int)prow[d_clip(0, W - 1, ix + j)];
-    }
-    atomicAdd(&cost[c], satd4x4_arr(d) * st);
-  }
-  __syncthreads();
-}
-
-/* Sub-pel cost at an even 1/8-pel vector without the quarter-pel planes
- * (k_me.h:247-258): the normative EIGHTTAP prediction of the block
- * (7.11.3, staged through LDS) and the SATD of all its 4x4 units. */
-template <int BW>
-DEVI int subpel_cost_pred(const Mav1FrameParams &fp, const uint8_t *srcL, const uint8_t *refY, int x, int y, int mvr,
-                          int mvc, uint8_t *pwin, int16_t *pmid, int lane) {
-  constexpr int WW = BW + 8, NR = BW / 4;
-  const int S = fp.stride[0], lastX = fp.frame_w - 1, lastY = fp.frame_h - 1;
-  const int posX = ((x << SUBPEL_BITS) + 2 * mvc) * 64 + 32, posY = ((y << SUBPEL_BITS) + 2 * mvr) * 64 + 32;
-  const int ix = posX >> 10, iy = posY >> 10;
-  const int16_t *kh = SUBPEL_FILTER(EIGHTTAP, (posX >> 6) & SUBPEL_MASK), *kv = SUBPEL_FILTER(EIGHTTAP, (posY >> 6) & SUBPEL_MASK);
-  __syncthreads();
-  for (int k = lane; k < (BW + 7) * (BW + 7); k += 64) {
-    const int r = k / (BW + 7), c = k - r * (BW + 7);
-    pwin[r * WW + c] = refY[d_clip(0, lastY, iy - 3 + r) * S + d_clip(0, lastX, ix - 3 + c)];
-  }
-  __syncthreads();
-  for (int k = lane; k < (BW + 7) * BW; k += 64) {
-    const int r = k / BW, c = k - r * BW;
-    const uint8_t *q = pwin + r * WW + c;
-    int acc = 0;
-#pragma unroll
-    for (int t = 0; t < 8; t++) acc += kh[t] * q[t];
-    pmid[k] = (int16_t)d_round2(acc, 3);
-  }
-  __syncthreads();
-  int s = 0;
-  for (int u = lane; u < NR * NR; u += 64) {
-    const int ucol = u % NR, urow = u / NR;
-    int d[16];
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const int r = urow * 4 + i, c = ucol * 4 + j;
-        int acc = 0;
-#pragma unroll
-        for (int t = 0; t < 8; t++) acc += kv[t] * pmid[(r + t) * BW + c];
-        d[4 * i + j] = (int)srcL[r * BW + c] - d_clip1(d_round2(acc, 11));
-      }
-    s += satd4x4_arr(d);
-  }
-  return wave_sum(s);
-}
-
-/* HP: sub-pel costs from the quarter-pel planes, else from predictions. */
+/* HP: sub-pel costs from the quarter-pel planes, else from predictions.
+ * One workgroup per (node, reference). Full-pel stages: ME_G lanes share a
+ * candidate, four samples per instruction, source, window and the decimated
+ * planes' windows staged in LDS. Sub-pel rings: a ring's candidates do not
+ * depend on each other, so the lanes take (candidate, 4x4 unit) pairs of the
+ * whole ring and the serial walk over the costs keeps its first minimum.
+ * Bound by the latency of the stages at small frames and by LDS reads and
+ * VALU issue at large ones. Levels 0 .. 3 at 352x288: 18, 7, 13 and 8 us
+ * (turbo), 58, 18, 25 and 22 us (full search); with one wave per node, a lane
+ * per candidate, byte loads and one prediction after another 100, 25, 19 and
+ * 10 us, 811, 123, 64 and 80 us. */
 template <int LEVEL, bool HP>
 DEVI void me_level_body(const Mav1FrameParams &fp, const uint8_t *__restrict__ src, const uint8_t *__restrict__ ref0, const uint8_t *__restrict__ ref1, const uint8_t *__restrict__ planes, long entryBytes, const uint8_t *__restrict__ srcDec, int32_t *__restrict__ field0, int32_t *__restrict__ field1, int nodesPerRef, const int blk_x, const int blk_y, const int blk_z) {
-  constexpr int BW = 64 >> LEVEL;
+  constexpr int BW = 64 >> LEVEL, NT = ME_NT<LEVEL>, NW = NT / 64, G = ME_G<LEVEL>, R = ME_WIN<LEVEL>;
   constexpr int N = 1 << LEVEL;
-  constexpr int WW = BW + 2 * WIN_R;
-  __shared__ uint8_t srcL[BW * BW];
-  __shared__ uint8_t win[WW * WW];
-  __shared__ uint8_t pwin[HP ? 1 : (BW + 7) * (BW + 8)];
-  __shared__ int16_t pmid[HP ? 1 : (BW + 7) * BW];
-  __shared__ int scost[9];
-  const int lane = threadIdx.x;
+  constexpr int WR = BW + (2 * R > 9 ? 2 * R : 9); /* window rows: full-pel radius R, or the predictions' support */
+  constexpr int WS = ((WR + 3) & ~3) + 4;          /* row stride: words, one more to read ahead */
+  constexpr int DN = BW / 4, DR = DN + 2 * ME_DEC_R, DS = ((DR + 3) & ~3) + 4;
+  __shared__ alignas(16) uint8_t srcL[BW * BW];
+  __shared__ alignas(16) uint8_t win[WR * WS + 16];
+  __shared__ alignas(16) uint8_t dsrc[LEVEL ? 4 : DN * DN], dwin[LEVEL ? 4 : DR * DS + 16];
+  __shared__ MeTaps taps;
+  __shared__ unsigned long long smin[2][NW];
+  __shared__ int scost[2][9];
+  const int tid = threadIdx.x, lane = tid & 63;
   const int r = blk_x / nodesPerRef, node = blk_x - r * nodesPerRef;
   const int sb = node >> (2 * LEVEL), i = node & (N * N - 1);
   const uint8_t *ref = r ? ref1 : ref0;
@@ -317,7 +330,7 @@ DEVI void me_level_body(const Mav1FrameParams &fp, const uint8_t *__restrict__ s
   m.y = (sb / fp.sb_cols) * 64 + (i / N) * BW;
   int32_t *out = field + (sb * MAV1_NUM_NODES + d_node_base(LEVEL) + i) * 2;
   if (m.x >= fp.frame_w || m.y >= fp.frame_h) {
-    if (lane == 0) out[0] = out[1] = 0;
+    if (tid == 0) out[0] = out[1] = 0;
     return;
   }
   m.range = fp.me_range;
@@ -343,16 +356,26 @@ DEVI void me_level_body(const Mav1FrameParams &fp, const uint8_t *__restrict__ s
   if (LEVEL == 3 && TB(fp, MAV1_T_ME_L3SUB)) m.nstage = 0;
   if (r && LEVEL == 3 && TB(fp, MAV1_T_ME_G3COPY) && fp.leaf && !fp.frame_is_intra) m.copy = 1;
   if (m.copy) {
-    if (lane == 0) {
+    if (tid == 0) {
       out[0] = m.pr;
       out[1] = m.pc;
     }
     return;
   }
-  const int S = fp.stride[0];
+  const int S = fp.stride[0], H1 = fp.frame_h - 1, W1 = fp.frame_w - 1;
   const uint8_t *srcY = src + fp.offset[0], *refY = ref + fp.offset[0];
-  for (int k = lane; k < BW * BW; k += 64) srcL[k] = srcY[(m.y + k / BW) * S + m.x + (k % BW)];
-  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < BW * BW / NT; k++) {
+    const int q = tid + k * NT;
+    srcL[q] = srcY[(m.y + q / BW) * S + m.x + (q % BW)];
+  }
+  if constexpr (!HP) me_taps(taps, tid);
+  /* the reference around (y, x) into the window: rows x cols samples, clamped */
+  auto stage = [&](int y, int x, int n) {
+    const int c0 = tid & 63;
+    for (int wr = tid >> 6; wr < n; wr += NW)
+      for (int wc = c0; wc < n; wc += 64) win[wr * WS + wc] = refY[d_clip(0, H1, y + wr) * S + d_clip(0, W1, x + wc)];
+  };
 
   int by = 0, bx = 0;
   for (int stg = 0; stg < m.nstage; stg++) {
@@ -370,35 +393,55 @@ DEVI void me_level_body(const Mav1FrameParams &fp, const uint8_t *__restrict__ s
     const int side = 2 * (m.range / m.step) + 1, count = 1 + side * side;
     const bool dec = TB(fp, MAV1_T_ME_DEC) && m.step >= 4;
     const int rs = (TB(fp, MAV1_T_ME_RSUB) && m.step == 1) ? 2 : 1;
-    const bool lds = !dec && m.range <= WIN_R;
-    const int oy0 = m.cy - m.range, ox0 = m.cx - m.range, wdim = BW + 2 * m.range;
-    if (lds) {
-      for (int k = lane; k < wdim * wdim; k += 64) {
-        int wr = k / wdim, wc = k - wr * wdim;
-        win[wr * WW + wc] = refY[d_clip(0, fp.frame_h - 1, m.y + oy0 + wr) * S + d_clip(0, fp.frame_w - 1, m.x + ox0 + wc)];
+    const bool lds = m.range <= (dec ? (LEVEL ? -1 : 4 * ME_DEC_R) : R);
+    const int oy0 = m.cy - m.range, ox0 = m.cx - m.range;
+    if (stg) __syncthreads(); /* the last stage's reads of the windows */
+    if constexpr (LEVEL == 0) {
+      if (dec && lds) {
+        const int W = (fp.frame_w + 3) >> 2, H = (fp.frame_h + 3) >> 2, x0 = m.x >> 2, y0 = m.y >> 2;
+        const int oy = oy0 >> 2, ox = ox0 >> 2, n = DN + 2 * (m.range >> 2);
+        if (tid < DN * DN) dsrc[tid] = srcDec[(size_t)d_min(y0 + tid / DN, H - 1) * W + d_min(x0 + tid % DN, W - 1)];
+        for (int wr = tid >> 5; wr < n; wr += NT / 32) /* n <= 32 */
+          if ((tid & 31) < n)
+            dwin[wr * DS + (tid & 31)] =
+                refDec[(size_t)d_clip(0, H - 1, y0 + oy + wr) * W + d_clip(0, W - 1, x0 + ox + (tid & 31))];
       }
-      __syncthreads();
     }
+    if (!dec && lds) stage(m.y + oy0, m.x + ox0, BW + 2 * m.range);
+    __syncthreads();
     unsigned long long best = ~0ull;
-    for (int k = lane; k < count; k += 64) {
+    const int g = tid & (G - 1);
+    for (int k = tid / G; k < ((count + NT / G - 1) & ~(NT / G - 1)); k += NT / G) {
       int dy, dx;
-      me_cand(m, k, dy, dx);
-      int rate = fp.ac_q[0] * me_bits(dy, dx) / 64, c;
-      if (dec)
-        c = sad_dec<BW>(fp, srcDec, refDec, m.x, m.y, dy, dx);
-      else if (lds)
-        c = sad_lds<BW>(srcL, win, WW, dy - oy0, dx - ox0, rs);
-      else
-        c = sad_global<BW>(fp, srcL, refY, m.x, m.y, dy, dx, rs);
-      unsigned long long key = pack_key(c + rate, k);
+      const int kk = d_min(k, count - 1);
+      me_cand(m, kk, dy, dx);
+      const int rate = fp.ac_q[0] * me_bits(dy, dx) / 64;
+      int c;
+      if (dec) {
+        if (LEVEL == 0 && lds)
+          c = sad_rows<DN, DS>(dsrc, dwin, (dy - oy0) >> 2, (dx - ox0) >> 2, g, G);
+        else
+          c = sad_rows_dec_global<BW>(fp, srcDec, refDec, m.x, m.y, dy, dx, g, G);
+        c *= 16;
+      } else if (lds) {
+        c = sad_rows<BW, WS>(srcL, win, dy - oy0, dx - ox0, g * rs, G * rs) * rs;
+      } else {
+        c = sad_rows_global<BW>(fp, srcL, refY, m.x, m.y, dy, dx, g * rs, G * rs) * rs;
+      }
+      const unsigned long long key = pack_key(me_group_sum<G>(c) + rate, kk);
       best = key < best ? key : best;
     }
     best = wave_min_u64(best);
+    if constexpr (NW > 1) {
+      if (lane == 0) smin[stg & 1][tid >> 6] = best;
+      __syncthreads();
+#pragma unroll
+      for (int w = 0; w < NW; w++) best = smin[stg & 1][w] < best ? smin[stg & 1][w] : best;
+    }
     me_cand(m, (int)(best & 0xffffffffu), by, bx);
-    __syncthreads();
   }
   if (LEVEL > 0 && TB(fp, MAV1_T_ME_KEEP) && by == m.cy && bx == m.cx) {
-    if (lane == 0) {
+    if (tid == 0) {
       out[0] = m.pr;
       out[1] = m.pc;
     }
@@ -407,73 +450,88 @@ DEVI void me_level_body(const Mav1FrameParams &fp, const uint8_t *__restrict__ s
   /* sub-pel refinement: half-pel ring, then quarter-pel ring unless
    * T_ME_HALF01 stops nodes >= 32 wide at half-pel */
   int mvr = m.nstage ? by * 8 : m.pr, mvc = m.nstage ? bx * 8 : m.pc;
-  const int st = (TB(fp, MAV1_T_ME_USUB) && BW >= 32) ? 2 : 1;
-  auto subpel = [&](int r_, int c_) {
-    if constexpr (HP) return subpel_cost_hp<BW>(fp, srcL, pl, m.x, m.y, r_, c_, st, lane);
-    else return subpel_cost_pred<BW>(fp, srcL, refY, m.x, m.y, r_, c_, pwin, pmid, lane);
-  };
+  constexpr int NR = BW / 4;
+  const int st = (HP && TB(fp, MAV1_T_ME_USUB) && BW >= 32) ? 2 : 1, nue = NR * NR / st;
   const int minStep = (BW >= 32 && TB(fp, MAV1_T_ME_HALF01)) ? 4 : 2;
   const bool cross = TB(fp, MAV1_T_ME_CROSS);
-  if constexpr (HP) {
-    /* The ring's costs do not depend on each other: all of a ring at once
-     * (the centre with the first ring), then the serial walk over them in
-     * ring order with the strict <, which keeps its first minimum. */
-    int bestS = 0;
-    for (int step = 4; step >= minStep; step >>= 1) {
-      const int cr0 = mvr, cc0 = mvc, first = step == 4;
-      int vr[9], vc[9], n = 0;
-      if (first) {
-        vr[0] = cr0;
-        vc[0] = cc0;
-        n = 1;
-      }
-#pragma unroll
-      for (int j = 0; j < 8; j++) {
-        if (cross && !(j == 1 || j == 3 || j == 4 || j == 6)) continue;
-        vr[n] = cr0 + (j < 3 ? -1 : j < 5 ? 0 : 1) * step;
-        vc[n] = cc0 + ((j == 0 || j == 3 || j == 5) ? -1 : (j == 1 || j == 6) ? 0 : 1) * step;
-        n++;
-      }
-      subpel_costs_hp<BW>(fp, srcL, pl, m.x, m.y, vr, vc, n, st, lane, scost);
-      if (first) bestS = scost[0];
-      for (int k = first; k < n; k++) {
-        const int c = scost[k];
-        if (c < bestS) {
-          bestS = c;
-          mvr = vr[k];
-          mvc = vc[k];
-        }
-      }
-      __syncthreads();
-    }
-    if (lane == 0) {
-      out[0] = mvr;
-      out[1] = mvc;
-    }
-    return;
+  /* the predictions' support around every vector the two rings can reach */
+  const int wy0 = ((mvr - 6) >> 3) - 3, wx0 = ((mvc - 6) >> 3) - 3;
+  if constexpr (!HP) {
+    __syncthreads();
+    stage(m.y + wy0, m.x + wx0, BW + 9);
   }
-  int bestS = subpel(mvr, mvc);
+  int bestS = 0;
   for (int step = 4; step >= minStep; step >>= 1) {
-    const int cr = mvr, cc = mvc;
-    for (int j = 0; j < (cross ? 4 : 8); j++) {
-      int k = cross ? (j == 0 ? 1 : j == 1 ? 3 : j == 2 ? 4 : 6) : j;
-      int dr = (k < 3 ? -1 : k < 5 ? 0 : 1) * step;
-      int dc = ((k == 0 || k == 3 || k == 5) ? -1 : (k == 1 || k == 6) ? 0 : 1) * step;
-      int c = subpel(cr + dr, cc + dc);
+    const int cr0 = mvr, cc0 = mvc, first = step == 4, ring = cross ? 4 : 8, n = first + ring;
+    /* candidate k: the centre (first ring), then the ring in its order */
+    auto vec = [&](int k, int &vr, int &vc) {
+      const int q = k - first, j = cross ? (q == 0 ? 1 : q == 1 ? 3 : q == 2 ? 4 : 6) : q;
+      vr = cr0 + (q < 0 ? 0 : j < 3 ? -1 : j < 5 ? 0 : 1) * step;
+      vc = cc0 + (q < 0 ? 0 : (j == 0 || j == 3 || j == 5) ? -1 : (j == 1 || j == 6) ? 0 : 1) * step;
+    };
+    int *cost = scost[first];
+    if (tid < n) cost[tid] = 0;
+    __syncthreads();
+    for (int p = tid; p < n * nue; p += NT) {
+      const int c = p / nue, u = (p - c * nue) * st;
+      int vr, vc;
+      vec(c, vr, vc);
+      const int ucol = u % NR, urow = u / NR;
+      uint32_t sw[4];
+#pragma unroll
+      for (int q = 0; q < 4; q++) sw[q] = *(const lds_cu32 *)(srcL + (urow * 4 + q) * BW + ucol * 4);
+      int d[16];
+      if constexpr (HP) {
+        const int W = fp.frame_w, iy = m.y + urow * 4 + (vr >> 3), ix = m.x + ucol * 4 + (vc >> 3);
+        const uint8_t *base = pl + (size_t)(((vr >> 1) & 3) * 4 + ((vc >> 1) & 3)) * W * fp.frame_h;
+        uint32_t pw[4];
+        if (ix >= 0 && ix + 3 < W) {
+#pragma unroll
+          for (int q = 0; q < 4; q++) __builtin_memcpy(&pw[q], base + (size_t)d_clip(0, H1, iy + q) * W + ix, 4);
+        } else {
+#pragma unroll
+          for (int q = 0; q < 4; q++) {
+            const uint8_t *prow = base + (size_t)d_clip(0, H1, iy + q) * W;
+            pw[q] = prow[d_clip(0, W1, ix)] | (uint32_t)prow[d_clip(0, W1, ix + 1)] << 8 |
+                    (uint32_t)prow[d_clip(0, W1, ix + 2)] << 16 | (uint32_t)prow[d_clip(0, W1, ix + 3)] << 24;
+          }
+        }
+#pragma unroll
+        for (int q = 0; q < 16; q++)
+          d[q] = (int)((sw[q >> 2] >> (8 * (q & 3))) & 255) - (int)((pw[q >> 2] >> (8 * (q & 3))) & 255);
+      } else {
+        me_pred_diff<WS>(taps, win, urow * 4 + (vr >> 3) - wy0, ucol * 4 + (vc >> 3) - wx0, (vr >> 1) & 3, (vc >> 1) & 3,
+                         sw, d);
+      }
+      /* the lanes of a quad or a row of 16 have the same candidate */
+      int s = satd4x4_arr(d) * st;
+      s += dpp_t<DPP_QX1>(s);
+      s += dpp_t<DPP_QX2>(s);
+      if constexpr (BW >= 16) {
+        s += dpp_t<DPP_HMIRROR>(s);
+        s += dpp_t<DPP_MIRROR>(s);
+        if ((lane & 15) == 0) atomicAdd(&cost[c], s);
+      } else {
+        if ((lane & 3) == 0) atomicAdd(&cost[c], s);
+      }
+    }
+    __syncthreads();
+    if (first) bestS = cost[0];
+    for (int k = first; k < n; k++) {
+      const int c = cost[k];
       if (c < bestS) {
         bestS = c;
-        mvr = cr + dr;
-        mvc = cc + dc;
+        vec(k, mvr, mvc);
       }
     }
   }
-  if (lane == 0) {
+  if (tid == 0) {
     out[0] = mvr;
     out[1] = mvc;
   }
 }
 template <int LEVEL, bool HP>
-__global__ __launch_bounds__(64) void k_me_level(const Mav1FrameParams fp, const uint8_t *__restrict__ src,
+__global__ __launch_bounds__(ME_NT<LEVEL>) void k_me_level(const Mav1FrameParams fp, const uint8_t *__restrict__ src,
                                                  const uint8_t *__restrict__ ref0, const uint8_t *__restrict__ ref1,
                                                  const uint8_t *__restrict__ planes, long entryBytes,
                                                  const uint8_t *__restrict__ srcDec, int32_t *__restrict__ field0,
@@ -487,10 +545,10 @@ static void launch_level(hipStream_t st, bool hp, dim3 grid, const Mav1FramePara
                          const uint8_t *ref0, const uint8_t *ref1, const uint8_t *planes, long entryBytes,
                          const uint8_t *srcDec, int32_t *field0, int32_t *field1, int nodesPerRef) {
   if (hp)
-    hipLaunchKernelGGL((k_me_level<LEVEL, true>), grid, dim3(64), 0, st, fp, src, ref0, ref1, planes, entryBytes, srcDec,
+    hipLaunchKernelGGL((k_me_level<LEVEL, true>), grid, dim3(ME_NT<LEVEL>), 0, st, fp, src, ref0, ref1, planes, entryBytes, srcDec,
                        field0, field1, nodesPerRef);
   else
-    hipLaunchKernelGGL((k_me_level<LEVEL, false>), grid, dim3(64), 0, st, fp, src, ref0, ref1, planes, entryBytes,
+    hipLaunchKernelGGL((k_me_level<LEVEL, false>), grid, dim3(ME_NT<LEVEL>), 0, st, fp, src, ref0, ref1, planes, entryBytes,
                        srcDec, field0, field1, nodesPerRef);
 }
 
@@ -548,7 +606,7 @@ hipError_t launch_dec_build_b(hipStream_t st, const BatchFrame *T, const BatchFr
 }
 
 template <int LEVEL, bool HP>
-__global__ __launch_bounds__(64) void k_me_level_b(const BatchFrame *__restrict__ T, const BatchGrid g) {
+__global__ __launch_bounds__(ME_NT<LEVEL>) void k_me_level_b(const BatchFrame *__restrict__ T, const BatchGrid g) {
   const BatchIdx b = batch_idx(g, xcd_item(blockIdx.x, gridDim.x, 1 << (2 * LEVEL)));
   const BatchFrame &F = T[b.f];
   me_level_body<LEVEL, HP>(F.fp, gptr(F.src), gptr(F.ref), gptr(F.gold), gptr(F.planes), (long)F.entry_bytes, gptr(F.planes) + 2 * F.entry_bytes,
@@ -558,9 +616,9 @@ __global__ __launch_bounds__(64) void k_me_level_b(const BatchFrame *__restrict_
 template <int LEVEL>
 static void launch_level_b(hipStream_t st, bool hp, const BatchFrame *T, const BatchGrid &g) {
   if (hp)
-    hipLaunchKernelGGL((k_me_level_b<LEVEL, true>), dim3(g.start[g.n]), dim3(64), 0, st, T, g);
+    hipLaunchKernelGGL((k_me_level_b<LEVEL, true>), dim3(g.start[g.n]), dim3(ME_NT<LEVEL>), 0, st, T, g);
   else
-    hipLaunchKernelGGL((k_me_level_b<LEVEL, false>), dim3(g.start[g.n]), dim3(64), 0, st, T, g);
+    hipLaunchKernelGGL((k_me_level_b<LEVEL, false>), dim3(g.start[g.n]), dim3(ME_NT<LEVEL>), 0, st, T, g);
 }
 
 hipError_t launch_me_level_b(hipStream_t st, int level, const BatchFrame *T, const BatchFrame *H, int n, int nref) {
