@@ -3,20 +3,21 @@
  *
  * Pass 1: one workgroup per table item (superblock, node, slot), one launch
  * per level (a node's depth pruning reads its ancestors' costs): four waves
- * for the 64x64 items, two for the 32x32 ones, a wave64 for the smaller ones. The item's
- * source block (luma + both chroma planes) is staged in LDS; inter
- * predictions run through an LDS reference window (8-tap horizontal pass
- * into int16 LDS rows, vertical pass into LDS bytes); intra predictions are
- * produced per sample inside the SATD loop from LDS edge arrays. 4x4 units
- * are spread over the threads and every SATD is a workgroup reduction, so
- * each cost is a uniform value and the mode decisions (first minimum, ties
- * as the serial code) are taken identically by all threads.
+ * for the 64x64 items, two for the 32x32 ones, a wave64 for the smaller ones.
+ * The item's source block (luma + both chroma planes) and the reference
+ * windows of its inter predictions are staged in LDS. Lanes take pairs of a
+ * candidate (an intra mode with its angle, a reference, a chroma-from-luma
+ * alpha) and a 4x4 unit, predict the unit in registers and add its SATD to
+ * the candidate's sum in LDS; the mode decisions (first minimum, ties as the
+ * serial code) are then taken identically by all threads.
  *
  * Pass 2: one wave per superblock runs the bottom-up partition choice over
  * the 85 nodes (lanes over the nodes of a level) and writes the blocks in
  * decode order (lanes over the 64 Z-order positions, prefix-scanned).
  */
 #include "dev_pred.h"
+
+#include <climits>
 #include "internal.h"
 
 #define TB(fp, bit) (((fp).turbo & (bit)) != 0)
@@ -106,16 +107,55 @@ int analysis_level_slots(const Mav1FrameParams &fp, int level) {
 
 template <int BW>
 struct AnaLds {
-  uint8_t srcY[BW * BW];
-  uint8_t srcC[2][(BW / 2) * (BW / 2)];
-  uint8_t pa[BW * BW];
-  uint8_t pb[BW * BW];
-  uint8_t win[(BW + 7) * (BW + 8)];
-  int16_t mid[(BW + 7) * BW];
-  int edge[3][2][EDGE_NEG + 2 * BW + 8]; /* [plane][above, left] */
+  static constexpr int WY = BW + 12, WC = BW / 2 + 12; /* window rows: support and words read ahead */
+  static constexpr int WIN_C = (BW + 7) * WY, WIN_P = (BW / 2 + 7) * WC;
+  alignas(4) uint8_t srcY[BW * BW];
+  alignas(4) uint8_t srcC[2][(BW / 2) * (BW / 2)];
+  alignas(4) uint8_t win[2][WIN_C + 2 * WIN_P + 4]; /* per reference: luma, U, V */
+  InterTaps taps[2][2];                             /* per reference: luma, chroma */
+  int edge[3][2][EDGE_NEG + 2 * BW + 8];            /* [plane][above, left] */
   int dcp[BW / 2 * BW / 2];
+  int satd[16]; /* per candidate mode */
+  int sse[2][33]; /* per plane and alpha + 16 */
 };
+/* v added into *to for the lanes of a unit count 1 << lu (a candidate's units
+ * are consecutive lanes). */
+DEVI void ana_add(int *to, int v, int lu, int lane) {
+  if (lu >= 2) {
+    v += dpp_t<DPP_QX1>(v);
+    v += dpp_t<DPP_QX2>(v);
+  }
+  if (lu >= 4) {
+    v += dpp_t<DPP_HMIRROR>(v);
+    v += dpp_t<DPP_MIRROR>(v);
+  }
+  if ((lane & (lu >= 4 ? 15 : lu >= 2 ? 3 : 0)) == 0) atomicAdd(to, v);
+}
+/* SATD of candidate `mode` with delta over one unit. */
+DEVI int ana_intra(int mode, int delta, int lw, int lh, int dcv, const int *A, const int *L, const uint8_t *s, int st,
+                   int uy, int ux) {
+  IntraMode im;
+  intra_mode_setup(im, mode, delta, lw, lh);
+  im.dcv = dcv;
+  im.corner = A[-1];
+  int d[16];
+  uint32_t sw[4];
+  intra_unit(im, A, L, uy, ux, d);
+  unit_load(s + uy * 4 * st + ux * 4, st, sw);
+#pragma unroll
+  for (int k = 0; k < 16; k++) d[k] = (int)((sw[k >> 2] >> (8 * (k & 3))) & 255) - d[k];
+  return satd4x4_arr(d);
+}
 
+/* One workgroup per analysis item. The candidates of a step do not depend on
+ * each other, so the lanes take (candidate, 4x4 unit) pairs: an 8x8 block has
+ * four units of luma and one of each chroma plane, and candidate by candidate
+ * most lanes idled behind a reduction each. An inter unit is predicted in
+ * registers by both passes of the filter.
+ * Bound by latency at small frames, by VALU issue and LDS reads at large ones.
+ * Levels 0 .. 3, before and now: 352x288 full search 139, 187, 186, 137 -> 45,
+ * 51, 42, 25 us; 1920x1080 key frame 139, 200, 374, 1358 -> 45, 57, 71,
+ * 142 us; 204x116 turbo 61, 61, 57, 43 -> 31, 20, 19, 14 us. */
 template <int LEVEL>
 DEVI void analyze_level_body(const Mav1FrameParams &fp, const uint8_t *__restrict__ src, const uint8_t *__restrict__ ref, const uint8_t *__restrict__ gold, const int32_t *__restrict__ mvf, const int32_t *__restrict__ mvg, long long *__restrict__ costs, Mav1BlockInfo *__restrict__ infos, int nslots, const int8_t *__restrict__ prune, const int blk_x, const int blk_y, const int blk_z) {
   constexpr int BW = 64 >> LEVEL, N = 1 << LEVEL;
@@ -191,23 +231,46 @@ DEVI void analyze_level_body(const Mav1FrameParams &fp, const uint8_t *__restric
       gc = mvg[(sbIdx * MAV1_NUM_NODES + node) * 2 + 1];
     }
     const int want = fp.golden ? (fp.compound ? 3 : 2) : 1;
-    long long s0 = 0, s1 = 0, s2 = 0;
-    for (int pl = 0; pl < 3; pl++) {
-      const int sub = pl > 0, bx = x >> sub, by = y >> sub, bw = w >> sub, bh = h >> sub, S = fp.stride[pl];
-      const int st = sub ? BW / 2 : BW;
-      const uint8_t *sblk = sub ? L.srcC[pl - 1] : L.srcY;
-      const int usub = TB(fp, MAV1_T_ANA_USUB) && bw >= 32;
-      wave_predict_inter<NT>(ref + fp.offset[pl], S, fp.frame_w, fp.frame_h, bx, by, bw, bh, lr, lc, sub, EIGHTTAP, L.win,
-                         L.mid, L.pa, st, nullptr, 11, lane);
-      if (want > 1)
-        wave_predict_inter<NT>(gold + fp.offset[pl], S, fp.frame_w, fp.frame_h, bx, by, bw, bh, gr, gc, sub, EIGHTTAP,
-                           L.win, L.mid, L.pb, st, nullptr, 11, lane);
-      int a0, a1, a2;
-      wave_satd3<NT>(sblk, L.pa, L.pb, st, bw, bh, usub, want, lane, &a0, &a1, &a2);
-      s0 += a0;
-      s1 += a1;
-      s2 += a2;
+    if (lane < 4) {
+      const int g = lane >> 1, sub = lane & 1;
+      inter_taps(L.taps[g][sub], x >> sub, y >> sub, w >> sub, h >> sub, g ? gr : lr, g ? gc : lc, sub);
     }
+    __syncthreads();
+    for (int g = 0; g < (want > 1 ? 2 : 1); g++)
+      for (int pl = 0; pl < 3; pl++) {
+        const int sub = pl > 0;
+        inter_stage<NT>((g ? gold : ref) + fp.offset[pl], fp.stride[pl], ((fp.frame_w + sub) >> sub) - 1,
+                        ((fp.frame_h + sub) >> sub) - 1, L.taps[g][sub], w >> sub, h >> sub,
+                        L.win[g] + (pl ? AnaLds<BW>::WIN_C + (pl - 1) * AnaLds<BW>::WIN_P : 0),
+                        pl ? AnaLds<BW>::WC : AnaLds<BW>::WY, lane);
+      }
+    __syncthreads();
+    int a0 = 0, a1 = 0, a2 = 0;
+    const int nY = 1 << (lw + lh - 4), lC = clw + clh - 4, nC = 1 << lC;
+    for (int q = lane; q < nY + 2 * nC; q += NT) {
+      const int pl = q < nY ? 0 : 1 + ((q - nY) >> lC), u = pl ? (q - nY) & (nC - 1) : q;
+      const int lx = (pl ? clw : lw) - 2, uy = u >> lx, ux = u & ((1 << lx) - 1);
+      const int st = pl ? BW / 2 : BW, ws = pl ? AnaLds<BW>::WC : AnaLds<BW>::WY;
+      const int usub = TB(fp, MAV1_T_ANA_USUB) && lx >= 3; /* every second unit of planes 32 wide and wider */
+      if (usub && ((ux + uy) & 1)) continue;
+      const int at = (pl ? AnaLds<BW>::WIN_C + (pl - 1) * AnaLds<BW>::WIN_P : 0) + uy * 4 * ws + ux * 4;
+      uint32_t sw[4], p0[4], p1[4];
+      unit_load((pl ? L.srcC[pl - 1] : L.srcY) + uy * 4 * st + ux * 4, st, sw);
+      inter_unit(L.taps[0][pl > 0], L.win[0], ws, at, p0);
+      a0 += unit_satd(sw, p0) << usub;
+      if (want > 1) {
+        inter_unit(L.taps[1][pl > 0], L.win[1], ws, at, p1);
+        a1 += unit_satd(sw, p1) << usub;
+        if (want > 2) {
+#pragma unroll
+          for (int k = 0; k < 4; k++) p0[k] = avg4(p0[k], p1[k]);
+          a2 += unit_satd(sw, p0) << usub;
+        }
+      }
+    }
+    const long long s0 = group_sum<NT>(a0);
+    const long long s1 = want > 1 ? group_sum<NT>(a1) : 0;
+    const long long s2 = want > 2 ? group_sum<NT>(a2) : 0;
     interCost = s0 + (long long)lam * (4 + mv_bits8(lr, lc)) / 8;
     mvr = lr;
     mvc = lc;
@@ -244,13 +307,18 @@ DEVI void analyze_level_body(const Mav1FrameParams &fp, const uint8_t *__restric
   if (!skipIntra) {
     wave_intra_edges<NT>(src + fp.offset[0], fp.stride[0], x, y, w, h, x > 0, y > 0, 0, 0, maxXY, maxYY, AY, LY, lane);
     const int dcY = wave_intra_dc<NT>(AY, LY, w, h, lw, lh, x > 0, y > 0, lane);
+    const int lu = lw + lh - 4;
+    if (lane < 16) L.satd[lane] = 0;
+    __syncthreads();
+    for (int q = lane; q < 13 << lu; q += NT) {
+      const int m = q >> lu, u = q & ((1 << lu) - 1);
+      if (tIntra && m != DC_PRED && m != V_PRED && m != H_PRED && m != SMOOTH_PRED) continue;
+      ana_add(&L.satd[m], ana_intra(m, 0, lw, lh, dcY, AY, LY, L.srcY, BW, u >> (lw - 2), u & ((w >> 2) - 1)), lu, lane);
+    }
+    __syncthreads();
     for (int m = DC_PRED; m <= PAETH_PRED; m++) {
       if (tIntra && m != DC_PRED && m != V_PRED && m != H_PRED && m != SMOOTH_PRED) continue;
-      IntraMode im;
-      intra_mode_setup(im, m, 0, lw, lh);
-      im.dcv = dcY;
-      im.corner = AY[-1];
-      long long cst = wave_intra_satd<NT>(im, AY, LY, L.srcY, BW, lane) + (long long)lam * mode_bits8(m) / 8;
+      const long long cst = L.satd[m] + (long long)lam * mode_bits8(m) / 8;
       if (best < 0 || cst < best) {
         best = cst;
         bestMode = m;
@@ -259,16 +327,21 @@ DEVI void analyze_level_body(const Mav1FrameParams &fp, const uint8_t *__restric
   }
   if (skipIntra) best = 1ll << 40;
   if (bestMode >= V_PRED && bestMode <= D67_PRED && !fp.fast) {
-    for (int d = -MAX_ANGLE_DELTA; d <= MAX_ANGLE_DELTA; d++) {
-      if (!d) continue;
-      IntraMode im;
-      intra_mode_setup(im, bestMode, d, lw, lh);
-      im.corner = AY[-1];
-      im.dcv = 0;
-      long long cst = wave_intra_satd<NT>(im, AY, LY, L.srcY, BW, lane) + (long long)lam * (mode_bits8(bestMode) + 16) / 8;
+    const int lu = lw + lh - 4;
+    __syncthreads();
+    if (lane < 16) L.satd[lane] = 0;
+    __syncthreads();
+    for (int q = lane; q < (2 * MAX_ANGLE_DELTA) << lu; q += NT) {
+      const int k = q >> lu, u = q & ((1 << lu) - 1), d = k < MAX_ANGLE_DELTA ? k - MAX_ANGLE_DELTA : k - MAX_ANGLE_DELTA + 1;
+      ana_add(&L.satd[k], ana_intra(bestMode, d, lw, lh, 0, AY, LY, L.srcY, BW, u >> (lw - 2), u & ((w >> 2) - 1)), lu,
+              lane);
+    }
+    __syncthreads();
+    for (int k = 0; k < 2 * MAX_ANGLE_DELTA; k++) {
+      const long long cst = L.satd[k] + (long long)lam * (mode_bits8(bestMode) + 16) / 8;
       if (cst < best) {
         best = cst;
-        bestDelta = d;
+        bestDelta = k < MAX_ANGLE_DELTA ? k - MAX_ANGLE_DELTA : k - MAX_ANGLE_DELTA + 1;
       }
     }
   }
@@ -286,18 +359,26 @@ DEVI void analyze_level_body(const Mav1FrameParams &fp, const uint8_t *__restric
                        lane);
       dcC[pl] = wave_intra_dc<NT>(A, Lc, cw, ch, clw, clh, cx > 0, cy > 0, lane);
     }
+    const int lu = clw + clh - 4;
+    auto tried = [&](int m) {
+      if (m >= V_PRED && m <= D67_PRED && m != V_PRED && m != H_PRED && m != bestMode) return false;
+      return !tIntra || m == DC_PRED || m == V_PRED || m == H_PRED || m == SMOOTH_PRED;
+    };
+    __syncthreads();
+    if (lane < 16) L.satd[lane] = 0;
+    __syncthreads();
+    for (int q = lane; q < 26 << lu; q += NT) {
+      const int m = q >> (lu + 1), pl = (q >> lu) & 1, u = q & ((1 << lu) - 1);
+      if (!tried(m)) continue;
+      ana_add(&L.satd[m],
+              ana_intra(m, m == bestMode ? bestDelta : 0, clw, clh, pl ? dcC[1] : dcC[0], L.edge[1 + pl][0] + EDGE_NEG,
+                        L.edge[1 + pl][1] + EDGE_NEG, L.srcC[pl], BW / 2, u >> (clw - 2), u & ((cw >> 2) - 1)),
+              lu, lane);
+    }
+    __syncthreads();
     for (int m = DC_PRED; m <= PAETH_PRED; m++) {
-      if (m >= V_PRED && m <= D67_PRED && m != V_PRED && m != H_PRED && m != bestMode) continue;
-      if (tIntra && m != DC_PRED && m != V_PRED && m != H_PRED && m != SMOOTH_PRED) continue;
-      const int d = m == bestMode ? bestDelta : 0;
-      long long cst = (long long)lam * (m == DC_PRED ? 8 : 24) / 8;
-      for (int pl = 0; pl < 2; pl++) {
-        IntraMode im;
-        intra_mode_setup(im, m, d, clw, clh);
-        im.dcv = dcC[pl];
-        im.corner = L.edge[1 + pl][0][EDGE_NEG - 1];
-        cst += wave_intra_satd<NT>(im, L.edge[1 + pl][0] + EDGE_NEG, L.edge[1 + pl][1] + EDGE_NEG, L.srcC[pl], BW / 2, lane);
-      }
+      if (!tried(m)) continue;
+      const long long cst = L.satd[m] + (long long)lam * (m == DC_PRED ? 8 : 24) / 8;
       if (bestUv < 0 || cst < bestUv) {
         bestUv = cst;
         bestUvMode = m;
@@ -319,42 +400,53 @@ DEVI void analyze_level_body(const Mav1FrameParams &fp, const uint8_t *__restric
       L.dcp[q] = v;
       lsum += v;
     }
+    for (int q = lane; q < 66; q += NT) (&L.sse[0][0])[q] = 0;
     lsum = group_sum<NT>(lsum);
     const int avg = d_round2(lsum, clw + clh);
     __syncthreads();
+    /* a lane takes |alpha| of both signs and every PARTS-th sample */
+    constexpr int PARTS = NT / 17;
+    const int part = lane / 17, aa = lane - part * 17;
+    if (part < PARTS)
+      for (int pl = 0; pl < 2; pl++) {
+        const int dcv = dcC[pl];
+        int ep = 0, en = 0;
+        for (int q = part; q < nC; q += PARTS) {
+          const int sv = L.srcC[pl][(q >> clw) * (BW / 2) + (q & (cw - 1))];
+          const int v = d_round2signed(aa * (L.dcp[q] - avg), 6);
+          const int dp = d_clip1(dcv + v) - sv, dn = d_clip1(dcv - v) - sv;
+          ep += dp * dp;
+          en += dn * dn;
+        }
+        atomicAdd(&L.sse[pl][16 + aa], ep);
+        if (aa) atomicAdd(&L.sse[pl][16 - aa], en);
+      }
+    __syncthreads();
+    int bestA[2];
+#pragma unroll
     for (int pl = 0; pl < 2; pl++) {
-      const uint8_t *sC = L.srcC[pl];
-      const int dcv = dcC[pl];
-      long long bestS = -1;
-      int bestA = 0;
-      for (int a = -16; a <= 16; a++) {
-        int e = 0;
-        for (int q = lane; q < nC; q += NT) {
-          int yy = q >> clw, xx = q & (cw - 1);
-          int dd = d_clip1(dcv + d_round2signed(a * (L.dcp[q] - avg), 6)) - sC[yy * (BW / 2) + xx];
-          e += dd * dd;
-        }
-        long long sse = group_sum<NT>(e);
-        if (bestS < 0 || sse < bestS) {
-          bestS = sse;
-          bestA = a;
-        }
-      }
-      int acc = 0;
-      for (int u = lane; u < nC / 16; u += NT) {
-        int nx = cw >> 2, uy = u / nx, ux = u - uy * nx, dd[16];
-#pragma unroll
-        for (int ii = 0; ii < 4; ii++)
-#pragma unroll
-          for (int jj = 0; jj < 4; jj++) {
-            int q = (uy * 4 + ii) * cw + ux * 4 + jj;
-            int pv = d_clip1(dcv + d_round2signed(bestA * (L.dcp[q] - avg), 6));
-            dd[4 * ii + jj] = (int)sC[(uy * 4 + ii) * (BW / 2) + ux * 4 + jj] - pv;
-          }
-        acc += satd4x4_arr(dd);
-      }
-      cst += group_sum<NT>(acc);
+      /* the first minimum: an SSE of at most 256 samples leaves room for its index */
+      const int k = lane & 63, key = k < 33 ? L.sse[pl][k] << 6 | k : INT_MAX;
+      bestA[pl] = (-wave_max_dpp(-key) & 63) - 16;
     }
+    int acc = 0;
+    const int lC = clw + clh - 4;
+    for (int q = lane; q < 2 << lC; q += NT) {
+      const int pl = q >> lC, u = q & ((1 << lC) - 1), uy = u >> (clw - 2), ux = u & ((cw >> 2) - 1);
+      const int dcv = pl ? dcC[1] : dcC[0], al = pl ? bestA[1] : bestA[0];
+      const uint8_t *sC = L.srcC[pl];
+      int dd[16];
+#pragma unroll
+      for (int ii = 0; ii < 4; ii++)
+#pragma unroll
+        for (int jj = 0; jj < 4; jj++) {
+          const int e = (uy * 4 + ii) * cw + ux * 4 + jj;
+          const int pv = d_clip1(dcv + d_round2signed(al * (L.dcp[e] - avg), 6));
+          dd[4 * ii + jj] = (int)sC[(uy * 4 + ii) * (BW / 2) + ux * 4 + jj] - pv;
+        }
+      acc += satd4x4_arr(dd);
+    }
+    cst += group_sum<NT>(acc);
     if (cst < bestUv) {
       bestUv = cst;
       bestUvMode = UV_CFL_PRED;
