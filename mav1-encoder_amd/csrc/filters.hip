@@ -34,16 +34,46 @@ __global__ __launch_bounds__(64) void k_filter_info(const Mav1FrameParams fp, co
 
 /* ---- deblocking ---- */
 
-DEVI int lf_txsz(int info, int plane) {
+/* log2 of the transform block's width and height: of Max_Tx_Size_Rect split
+ * tx_depth times (a square into quarters, else across its longer side) in
+ * luma, of the uv transform size in chroma. By arithmetic on the block's
+ * size: table after table would be a chain of memory latencies. */
+DEVI void lf_txdim(int info, int plane, int &lw, int &lh) {
   const int bs = info & 31;
+  lw = Mi_Width_Log2[bs] + 2;
+  lh = Mi_Height_Log2[bs] + 2;
   if (plane) {
-    int t = Max_Tx_Size_Rect[SUBSAMPLED_SIZE(bs, 1, 1)];
-    if (Tx_Width[t] == 64 || Tx_Height[t] == 64) t = Tx_Width[t] == 16 ? TX_16X32 : Tx_Height[t] == 16 ? TX_32X16 : TX_32X32;
-    return t;
+    lw = d_clip(2, 5, lw - 1);
+    lh = d_clip(2, 5, lh - 1);
+    return;
   }
-  int t = Max_Tx_Size_Rect[bs];
-  for (int d = (info >> 6) & 3; d > 0; d--) t = Split_Tx_Size[t];
-  return t;
+  lw = d_min(6, lw);
+  lh = d_min(6, lh);
+  for (int d = (info >> 6) & 3; d > 0; d--) {
+    const int w = lw;
+    lw = d_max(2, lw - (lw >= lh));
+    lh = d_max(2, lh - (lh >= w));
+  }
+}
+
+/* The wide filter (7.14.6.4) of N samples on either side, the taps |j| <= N2
+ * counted twice. Unrolled, so that the samples stay in registers: with N and
+ * the taps at run time they went through scratch memory, and a pass over a
+ * 204x116 frame, bound by latency, took 31 us instead of 5.5 (with the size
+ * tables of lf_txdim in a chain before that). */
+template <int N, int N2, int LOG2>
+DEVI void lf_wide(const int (&p)[7], const int (&q)[7], uint8_t *s, int step) {
+#pragma unroll
+  for (int i = -N; i < N; i++) {
+    int t = 0;
+#pragma unroll
+    for (int j = -N; j <= N; j++) {
+      const int k = i + j < -(N + 1) ? -(N + 1) : i + j > N ? N : i + j;
+      const int v = k < 0 ? p[k < 0 ? -k - 1 : 0] : q[k < 0 ? 0 : k];
+      t += (j < 0 ? -j : j) <= N2 ? 2 * v : v;
+    }
+    s[i * step] = (uint8_t)d_round2(t, LOG2);
+  }
 }
 
 /* 7.14.6 at one sample position: s points at q0, step crosses the edge.
@@ -92,21 +122,9 @@ DEVI void lf_sample(uint8_t *s, int step, int plane, int lvl, int sharp, int siz
     }
     return;
   }
-  const int log2 = (size == 8 || !flat2) ? 3 : 4;
-  const int n = log2 == 4 ? 6 : plane == 0 ? 3 : 2;
-  const int n2 = (log2 == 3 && plane == 0) ? 0 : 1;
-  int v[14], out[12];
-#pragma unroll
-  for (int k = 0; k < 7; k++) {
-    v[6 - k] = p[k];
-    v[7 + k] = q[k];
-  }
-  for (int i = -n; i < n; i++) {
-    int t = 0;
-    for (int j = -n; j <= n; j++) t += v[d_clip(-(n + 1), n, i + j) + 7] * (d_abs(j) <= n2 ? 2 : 1);
-    out[i + n] = d_round2(t, log2);
-  }
-  for (int i = -n; i < n; i++) s[i * step] = (uint8_t)out[i + n];
+  if (size >= 16 && flat2) lf_wide<6, 1, 4>(p, q, s, step);
+  else if (plane == 0) lf_wide<3, 0, 3>(p, q, s, step);
+  else lf_wide<2, 1, 3>(p, q, s, step);
 }
 
 /* pass 0: x = vertical edge unit (4 samples), y = sample row;
@@ -134,10 +152,12 @@ DEVI void deblock_body(const Mav1FrameParams &fp, uint8_t *rec, const uint8_t *_
   if (pass == 0 ? x == 0 : y == 0) return;
   const int row = r0 | sub, col = c0 | sub, step = 1 << sub;
   const int pr = pass == 1 ? row - step : row, pc = pass == 0 ? col - step : col;
-  const int t = lf_txsz(info[row * fp.mi_cols + col], plane), tp = lf_txsz(info[pr * fp.mi_cols + pc], plane);
-  const int onEdge = pass == 0 ? ((x >> sub) & (Tx_Width[t] - 1)) == 0 : ((y >> sub) & (Tx_Height[t] - 1)) == 0;
-  if (!onEdge) return;
-  const int sz = pass == 0 ? d_min(Tx_Width[t], Tx_Width[tp]) : d_min(Tx_Height[t], Tx_Height[tp]);
+  int tw, th, pw, ph;
+  lf_txdim(info[row * fp.mi_cols + col], plane, tw, th);
+  lf_txdim(info[pr * fp.mi_cols + pc], plane, pw, ph);
+  const int lg = pass == 0 ? tw : th;
+  if (((pass == 0 ? x : y) >> sub) & ((1 << lg) - 1)) return;
+  const int sz = 1 << d_min(lg, pass == 0 ? pw : ph);
   const int S = fp.stride[plane];
   lf_sample(rec + fp.offset[plane] + sy * S + sx, pass == 0 ? 1 : S, plane, lvl, fp.lf_sharpness,
             d_min(plane ? 8 : 16, sz));
