@@ -89,7 +89,7 @@ def algorithmic_bytes(kernel, fp, nref):
         return F + 2 * F + mi  # turbo: two parameter sets written
     if kernel == "cdef_select":
         return 2 * F + F + F
-    if kernel == "lr_fit":
+    if kernel in ("lr_fit", "lr_path"):
         return 3 * F
     if kernel == "lr_chain":
         return 48 * sum(fp.lr_unit_rows[p] * fp.lr_unit_cols[p] for p in range(3))
@@ -176,8 +176,8 @@ def main():
 
     kernels = ["qpel_build", "dec_build", "me_level0", "me_level1", "me_level2", "me_level3", "analyze_level0",
                "analyze_level1", "analyze_level2", "analyze_level3", "analyze_table", "edge_types", "recon_inter",
-               "intra_sched", "recon_intra", "filter_info", "deblock", "cdef", "cdef_select", "lr_fit", "lr_chain",
-               "lr_apply"]
+               "intra_sched", "recon_intra", "filter_info", "deblock", "cdef", "cdef_select", "lr_fit", "lr_path",
+               "lr_chain", "lr_apply"]
 
     devname = [""]
 

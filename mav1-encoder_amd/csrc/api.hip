@@ -669,10 +669,18 @@ int mav1hip_launch_lr_select(mav1hip_ctx *c, int32_t lr_test) {
          return launch_lr_fit(c->stream, c->fp, c->b_src, c->d_rec, c->d_dbk, c->d_lrstats, c->lr_units);
        })))
     return rc;
-  return timed(c, "lr_chain", [&] {
-    return launch_lr_chain(c->stream, c->fp, c->b_src, c->d_rec, c->d_dbk, c->d_lrstats, c->d_lrunits, c->d_lrtype,
-                           lr_test != 0, c->d_lrreruns);
-  });
+  for (int last = 0; last < 2; last++) {
+    if (last && (rc = timed(c, "lr_path", [&] {
+                   return launch_lr_path(c->stream, c->fp, c->b_src, c->d_rec, c->d_dbk, c->d_lrstats, c->lr_units);
+                 })))
+      return rc;
+    if ((rc = timed(c, "lr_chain", [&] {
+           return launch_lr_chain(c->stream, c->fp, c->b_src, c->d_rec, c->d_dbk, c->d_lrstats, c->d_lrunits,
+                                  c->d_lrtype, lr_test != 0, c->d_lrreruns, last);
+         })))
+      return rc;
+  }
+  return MAV1HIP_OK;
 }
 
 int mav1hip_lr_select(mav1hip_ctx *c, const Mav1FrameParams *fp, const uint8_t *src, const uint8_t *cdef,

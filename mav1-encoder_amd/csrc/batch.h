@@ -125,7 +125,8 @@ hipError_t launch_cdef_select_b(hipStream_t st, const BatchFrame *T, const Batch
 hipError_t launch_lr_apply_b(hipStream_t st, const BatchFrame *T, const BatchFrame *H, int n);
 hipError_t launch_decision_grid_b(hipStream_t st, const BatchFrame *T, const BatchFrame *H, int n);
 hipError_t launch_lr_fit_b(hipStream_t st, const BatchFrame *T, const BatchFrame *H, int n);
-hipError_t launch_lr_chain_b(hipStream_t st, const BatchFrame *T, int n, int lrTest);
+hipError_t launch_lr_path_b(hipStream_t st, const BatchFrame *T, const BatchFrame *H, int n);
+hipError_t launch_lr_chain_b(hipStream_t st, const BatchFrame *T, int n, int lrTest, int last);
 /* Frame copies and clears of the driver: which 0 = reconstruction into the
  * deblocked copy, 1 = reconstruction into the restoration output, 2 = the
  * CDEF choices cleared. */

@@ -74,10 +74,14 @@ size_t lr_stat_bytes();
 /* The fit of every unit with its refinement under the default reference. */
 hipError_t launch_lr_fit(hipStream_t st, const Mav1FrameParams &fp, const uint8_t *src, const uint8_t *cdef,
                          const uint8_t *dbk, void *stats, int nunits);
-/* The unit chains. */
+/* Refinement of the units from each plane's chain restart point on. */
+hipError_t launch_lr_path(hipStream_t st, const Mav1FrameParams &fp, const uint8_t *src, const uint8_t *cdef,
+                          const uint8_t *dbk, void *stats, int nunits);
+/* The unit chains; not last: they may end early, for launch_lr_path and a
+ * further launch. */
 hipError_t launch_lr_chain(hipStream_t st, const Mav1FrameParams &fp, const uint8_t *src, const uint8_t *cdef,
-                           const uint8_t *dbk, const void *stats, Mav1LrUnit *units, int *lrType, int lrTest,
-                           int *reruns);
+                           const uint8_t *dbk, void *stats, Mav1LrUnit *units, int *lrType, int lrTest, int *reruns,
+                           int last);
 
 /* api.hip: library-internal access to a context for the sequence driver */
 /* A context on two streams the caller keeps (neither created nor destroyed

@@ -13,7 +13,9 @@
  *               true references. The refinement's SSEs do not depend on the
  *               reference, so a unit's refinement is replayed from its
  *               recorded SSEs, and done again only if a step of the replay
- *               decides otherwise than the record.
+ *               decides otherwise than the record;
+ *   k_lr_path   one workgroup per unit: the refinement of the units left
+ *               after several such, between two launches of the chain.
  * The Wiener fit is FP64 and its rounded result decides the coded taps: it
  * accumulates in the reference's order (block by block, sample by sample,
  * one lane per accumulator) with the reference's operand order, and this
@@ -78,6 +80,13 @@ struct LrTrace {
   uint32_t cur[6], m[6], p[6];
 };
 
+/* Where a plane's chain stands between its launches. */
+struct LrChain {
+  int start; /* next unit (plane index) to decide */
+  int done, used, nrerun;
+  int ref[6], refX[2]; /* running references */
+};
+
 /* Per-unit search state between the kernels. */
 struct LrUnitStat {
   uint32_t sseNone;
@@ -86,6 +95,7 @@ struct LrUnitStat {
   int w0[6];    /* fitted Wiener taps: [pass * 3 + j] */
   int wStar[6]; /* the taps the refinement arrived at */
   LrTrace tr;
+  LrChain chain; /* of the plane, in its first unit */
 };
 
 DEVI int lr_stripe_row(int k, int sub) { return (64 * k - 8) >> sub; }
@@ -1128,6 +1138,12 @@ DEVI void lr_fit_body(const Mav1FrameParams &fp, const uint8_t *__restrict__ src
     return;
   }
   lr_bits_init(tid);
+  if (tid == 0 && u == fp.lr_unit_off[g.p]) {
+    LrChain c = {};
+    for (int k = 0; k < 6; k++) c.ref[k] = Wiener_Taps_Mid[k % 3];
+    for (int k = 0; k < 2; k++) c.refX[k] = Sgrproj_Xqd_Mid[k];
+    st.chain = c;
+  }
   int w[6];
   const uint32_t sseNone = g.p ? lr_wiener_fit<2, 2>(g, w, tid) : lr_wiener_fit<3, 4>(g, w, tid);
   int ref[6];
@@ -1147,19 +1163,47 @@ __global__ __launch_bounds__(LR_T) void k_lr_fit(const Mav1FrameParams fp, const
   lr_fit_body(fp, src, cdef, dbk, stats, blockIdx.x, blockIdx.y);
 }
 
+/* Per unit: the refinement under the plane's running reference, for the
+ * units from the chain's restart point on (none if it is done). */
+DEVI void lr_path_body(const Mav1FrameParams &fp, const uint8_t *__restrict__ src, const uint8_t *__restrict__ cdef, const uint8_t *__restrict__ dbk, LrUnitStat *__restrict__ stats, const int u) {
+  __shared__ LrUnitLds U;
+  const int tid = threadIdx.x, p = u < fp.lr_unit_off[1] ? 0 : u < fp.lr_unit_off[2] ? 1 : 2;
+  const LrChain &cs = stats[fp.lr_unit_off[p]].chain;
+  if (cs.done || u - fp.lr_unit_off[p] < cs.start) return;
+  LrGeo g;
+  lr_geo(fp, u, g);
+  lr_bits_init(tid);
+  lr_stage(fp, g, cdef, dbk, src, U, tid);
+  int w[6], ref[6];
+#pragma unroll
+  for (int k = 0; k < 6; k++) {
+    w[k] = stats[u].w0[k];
+    ref[k] = cs.ref[k];
+  }
+  LrTrace tr;
+  lr_refine(fp.lambda, g, U, w, ref, &tr, tid);
+  if (tid == 0) lr_record(stats[u], w, tr);
+}
+__global__ __launch_bounds__(LR_T) void k_lr_path(const Mav1FrameParams fp, const uint8_t *__restrict__ src,
+                                                  const uint8_t *__restrict__ cdef, const uint8_t *__restrict__ dbk,
+                                                  LrUnitStat *__restrict__ stats) {
+  lr_path_body(fp, src, cdef, dbk, stats, blockIdx.x);
+}
+
 /* Per plane, units in raster order with the true running references: the
  * choice of lr_select (lr_search.c:262-349). LR_CB units at a time are scored
  * side by side under the running references, two per wave (lr_score), and
  * accepted up to the first that changes a reference or whose refinement has
  * to run again; that one and the next such units are then refined, one per
- * LR_T threads, and scored anew. units[] and lrType[plane] receive the
- * result, reruns[plane] the number of refinements run here. The next units'
- * statistics are loaded ahead.
+ * LR_T threads, and scored anew. After maxSteps such steps the launch records
+ * where it stands and ends: references that change in a burst are followed
+ * here, and where units keep coming out otherwise, k_lr_path refines all that
+ * are left side by side under the reference then running, and the next launch
+ * goes on. units[] and lrType[plane] receive the result, reruns[plane] the
+ * number of refinements run here. The next units' statistics are loaded ahead.
  * Bound by the latency of a step, one per LR_CB units or change of a
  * reference, and by the refinements: 62 us for a 1920x1080 key frame, 240 us
- * with one thread accepting unit by unit in three launches; 2.7 ms for
- * 1920x1080 planes of noise whose references change all the time, 15 ms with
- * a refinement in place of every replay. */
+ * with one thread accepting unit by unit in three launches. */
 #define LR_CB 16
 #define LR_CT 512 /* 32 threads per unit; the refinement takes about 200 registers */
 #define LR_CG (LR_CT / LR_T)
@@ -1273,10 +1317,13 @@ DEVI void lr_accept(LrWalk &W, int p, int li, int nb, int lane) {
   }
 }
 
-DEVI void lr_chain_body(const Mav1FrameParams &fp, const uint8_t *__restrict__ src, const uint8_t *__restrict__ cdef, const uint8_t *__restrict__ dbk, const LrUnitStat *__restrict__ stats, Mav1LrUnit *__restrict__ units, int *__restrict__ lrType, int lrTest, int *__restrict__ reruns, const int p) {
+DEVI void lr_chain_body(const Mav1FrameParams &fp, const uint8_t *__restrict__ src, const uint8_t *__restrict__ cdef, const uint8_t *__restrict__ dbk, LrUnitStat *__restrict__ stats, Mav1LrUnit *__restrict__ units, int *__restrict__ lrType, int lrTest, int *__restrict__ reruns, int maxSteps, const int p) {
   const int tid = threadIdx.x;
   __shared__ LrWalk W;
   const int nu = fp.lr_unit_rows[p] * fp.lr_unit_cols[p], off = fp.lr_unit_off[p];
+  LrChain &cs = stats[off].chain;
+  if (cs.done) return;
+  const int b00 = cs.start;
   constexpr int SW = (int)(sizeof(LrUnitStat) / 4), NV = (LR_CB * SW + LR_CT - 1) / LR_CT;
   int v[NV]; /* the next batch's statistics */
   auto fetch = [&](int b0) {
@@ -1286,20 +1333,22 @@ DEVI void lr_chain_body(const Mav1FrameParams &fp, const uint8_t *__restrict__ s
       if (tid + i * LR_CT < words) v[i] = ((const int *)(stats + off + b0))[tid + i * LR_CT];
   };
   lr_bits_init(tid);
-  if (tid < 6) W.ref[tid] = Wiener_Taps_Mid[tid % 3];
-  if (tid < 2) W.refX[tid] = Sgrproj_Xqd_Mid[tid];
-  if (tid == 0) W.used = 0;
+  if (tid < 6) W.ref[tid] = cs.ref[tid];
+  if (tid < 2) W.refX[tid] = cs.refX[tid];
+  if (tid == 0) W.used = cs.used;
   for (int q = tid; q < LR_CB * (int)(sizeof(Mav1LrUnit) / 4); q += LR_CT) ((int *)W.un)[q] = 0; /* padding included */
-  int nrerun = 0;
-  fetch(0);
-  for (int b0 = 0; b0 < nu; b0 += LR_CB) {
+  int nrerun = cs.nrerun, steps = 0;
+  fetch(b00);
+  for (int b0 = b00; b0 < nu; b0 += LR_CB) {
     const int nb = d_min(LR_CB, nu - b0);
 #pragma unroll
     for (int i = 0; i < NV; i++)
       if (tid + i * LR_CT < nb * SW) ((int *)W.st)[tid + i * LR_CT] = v[i];
     if (b0 + LR_CB < nu) fetch(b0 + LR_CB);
     __syncthreads();
-    for (int li = 0; li < nb;) {
+    int li = 0;
+    bool stop = false;
+    while (li < nb) {
       const int u = li + (tid >> 5);
       if (d_uni(tid >> 6) * 2 + li < nb) /* a wave's second unit may lie past the end: the last one once more */
         lr_score(fp.lambda, W, p, d_min(u, nb - 1), (b0 + d_min(u, nb - 1)) & 1, lrTest, tid & 63);
@@ -1309,6 +1358,10 @@ DEVI void lr_chain_body(const Mav1FrameParams &fp, const uint8_t *__restrict__ s
       li = W.next;
       const int nre = W.nre;
       if (!nre) continue;
+      if (steps++ == maxSteps) {
+        stop = true;
+        break;
+      }
       /* units again, under the running reference; then they are scored anew */
       const int grp = d_uni(tid / LR_T), t = tid % LR_T, ru = W.re[d_min(grp, nre - 1)];
       LrUnitLds &U = W.re_[grp];
@@ -1328,20 +1381,32 @@ DEVI void lr_chain_body(const Mav1FrameParams &fp, const uint8_t *__restrict__ s
       nrerun += nre;
       __syncthreads();
     }
-    for (int q = tid; q < nb * (int)(sizeof(Mav1LrUnit) / 4); q += LR_CT)
+    for (int q = tid; q < li * (int)(sizeof(Mav1LrUnit) / 4); q += LR_CT)
       ((int *)(units + off + b0))[q] = ((const int *)W.un)[q];
+    if (stop) {
+      if (tid == 0) {
+        cs.start = b0 + li;
+        cs.used = W.used;
+        cs.nrerun = nrerun;
+        for (int k = 0; k < 6; k++) cs.ref[k] = W.ref[k];
+        for (int k = 0; k < 2; k++) cs.refX[k] = W.refX[k];
+      }
+      return;
+    }
     __syncthreads();
   }
   if (tid == 0) {
+    cs.done = 1;
     lrType[p] = W.used ? RESTORE_SWITCHABLE : RESTORE_NONE;
     reruns[p] = nrerun;
   }
 }
 __global__ __launch_bounds__(LR_CT) void k_lr_chain(const Mav1FrameParams fp, const uint8_t *__restrict__ src,
                                                     const uint8_t *__restrict__ cdef, const uint8_t *__restrict__ dbk,
-                                                    const LrUnitStat *__restrict__ stats, Mav1LrUnit *__restrict__ units,
-                                                    int *__restrict__ lrType, int lrTest, int *__restrict__ reruns) {
-  lr_chain_body(fp, src, cdef, dbk, stats, units, lrType, lrTest, reruns, blockIdx.x);
+                                                    LrUnitStat *__restrict__ stats, Mav1LrUnit *__restrict__ units,
+                                                    int *__restrict__ lrType, int lrTest, int *__restrict__ reruns,
+                                                    int maxSteps) {
+  lr_chain_body(fp, src, cdef, dbk, stats, units, lrType, lrTest, reruns, maxSteps, blockIdx.x);
 }
 
 static_assert(sizeof(LrUnitStat) <= LR_STAT_MAX_BYTES, "LR_STAT_MAX_BYTES too small");
@@ -1353,11 +1418,20 @@ hipError_t launch_lr_fit(hipStream_t st, const Mav1FrameParams &fp, const uint8_
   return hipGetLastError();
 }
 
+/* Steps of a chain launch before the refinement pass. */
+#define LR_STEPS 4
+
+hipError_t launch_lr_path(hipStream_t st, const Mav1FrameParams &fp, const uint8_t *src, const uint8_t *cdef,
+                          const uint8_t *dbk, void *stats, int nunits) {
+  hipLaunchKernelGGL(k_lr_path, dim3(nunits), dim3(LR_T), 0, st, fp, src, cdef, dbk, (LrUnitStat *)stats);
+  return hipGetLastError();
+}
+
 hipError_t launch_lr_chain(hipStream_t st, const Mav1FrameParams &fp, const uint8_t *src, const uint8_t *cdef,
-                           const uint8_t *dbk, const void *stats, Mav1LrUnit *units, int *lrType, int lrTest,
-                           int *reruns) {
-  hipLaunchKernelGGL(k_lr_chain, dim3(3), dim3(LR_CT), 0, st, fp, src, cdef, dbk, (const LrUnitStat *)stats, units,
-                     lrType, lrTest, reruns);
+                           const uint8_t *dbk, void *stats, Mav1LrUnit *units, int *lrType, int lrTest, int *reruns,
+                           int last) {
+  hipLaunchKernelGGL(k_lr_chain, dim3(3), dim3(LR_CT), 0, st, fp, src, cdef, dbk, (LrUnitStat *)stats, units, lrType,
+                     lrTest, reruns, last ? INT_MAX : LR_STEPS);
   return hipGetLastError();
 }
 
@@ -1372,10 +1446,10 @@ __global__ __launch_bounds__(LR_T) void k_lr_fit_b(const BatchFrame *__restrict_
   const BatchFrame &F = T[b.f];
   lr_fit_body(F.fp, gptr(F.src), gptr(F.rec), gptr(F.dbk), (LrUnitStat *)gptr(F.lrstats), b.x, part);
 }
-__global__ __launch_bounds__(LR_CT) void k_lr_chain_b(const BatchFrame *__restrict__ T, int lrTest) {
+__global__ __launch_bounds__(LR_CT) void k_lr_chain_b(const BatchFrame *__restrict__ T, int lrTest, int maxSteps) {
   const BatchFrame &F = T[blockIdx.x / 3];
-  lr_chain_body(F.fp, gptr(F.src), gptr(F.rec), gptr(F.dbk), (const LrUnitStat *)gptr(F.lrstats), gptr(F.lrunits),
-                gptr(F.lrtype), lrTest, gptr(F.lrreruns), blockIdx.x % 3);
+  lr_chain_body(F.fp, gptr(F.src), gptr(F.rec), gptr(F.dbk), (LrUnitStat *)gptr(F.lrstats), gptr(F.lrunits),
+                gptr(F.lrtype), lrTest, gptr(F.lrreruns), maxSteps, blockIdx.x % 3);
 }
 
 static BatchGrid unit_grid(const BatchFrame *H, int n) {
@@ -1390,7 +1464,19 @@ hipError_t launch_lr_fit_b(hipStream_t st, const BatchFrame *T, const BatchFrame
   return hipGetLastError();
 }
 
-hipError_t launch_lr_chain_b(hipStream_t st, const BatchFrame *T, int n, int lrTest) {
-  hipLaunchKernelGGL(k_lr_chain_b, dim3(3 * n), dim3(LR_CT), 0, st, T, lrTest);
+__global__ __launch_bounds__(LR_T) void k_lr_path_b(const BatchFrame *__restrict__ T, const BatchGrid g) {
+  const BatchIdx b = batch_idx(g);
+  const BatchFrame &F = T[b.f];
+  lr_path_body(F.fp, gptr(F.src), gptr(F.rec), gptr(F.dbk), (LrUnitStat *)gptr(F.lrstats), b.x);
+}
+
+hipError_t launch_lr_path_b(hipStream_t st, const BatchFrame *T, const BatchFrame *H, int n) {
+  const BatchGrid g = unit_grid(H, n);
+  hipLaunchKernelGGL(k_lr_path_b, dim3(g.start[n]), dim3(LR_T), 0, st, T, g);
+  return hipGetLastError();
+}
+
+hipError_t launch_lr_chain_b(hipStream_t st, const BatchFrame *T, int n, int lrTest, int last) {
+  hipLaunchKernelGGL(k_lr_chain_b, dim3(3 * n), dim3(LR_CT), 0, st, T, lrTest, last ? INT_MAX : LR_STEPS);
   return hipGetLastError();
 }

@@ -95,7 +95,10 @@ int mav1hip_lr_select_static(const Mav1FrameParams *fp, const uint8_t *src, cons
   int *reruns = (int *)(d->ptr + kStatsBytes);
   hipStream_t st = (hipStream_t)stream;
   hipError_t e = launch_lr_fit(st, *fp, src, cdef, dbk, stats, n);
-  if (e == hipSuccess) e = launch_lr_chain(st, *fp, src, cdef, dbk, stats, units, lr_type, lr_test != 0, reruns);
+  for (int last = 0; last < 2 && e == hipSuccess; last++) {
+    if (last) e = launch_lr_path(st, *fp, src, cdef, dbk, stats, n);
+    if (e == hipSuccess) e = launch_lr_chain(st, *fp, src, cdef, dbk, stats, units, lr_type, lr_test != 0, reruns, last);
+  }
   if (e != hipSuccess) return fail(err, errlen, MAV1HIP_EDEVICE, "lr_select_static: launch", e);
   return MAV1HIP_OK;
 }

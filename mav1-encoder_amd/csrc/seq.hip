@@ -959,7 +959,9 @@ int round_late(mav1hip_batch *b, Round &R) {
     LCHK(b, "cdef choice clear", launch_frame_op_b(st, T, H, n, 2));
   if (pl.restoration) {
     LCHK(b, "lr_fit", launch_lr_fit_b(st, T, H, n));
-    LCHK(b, "lr_chain", launch_lr_chain_b(st, T, n, b->lr_test != 0));
+    LCHK(b, "lr_chain", launch_lr_chain_b(st, T, n, b->lr_test != 0, 0));
+    LCHK(b, "lr_path", launch_lr_path_b(st, T, H, n));
+    LCHK(b, "lr_chain", launch_lr_chain_b(st, T, n, b->lr_test != 0, 1));
     LCHK(b, "restoration copy", launch_frame_op_b(st, T, H, n, 1));
     LCHK(b, "lr_apply", launch_lr_apply_b(st, T, H, n));
   }
