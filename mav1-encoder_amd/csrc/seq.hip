@@ -832,7 +832,7 @@ Sig sig_of(const mav1hip_seq *s, const Frame &f) {
                    f.fp.golden,        f.fp.turbo,        f.plan.filter_info,
                    f.plan.deblock,     f.plan.cdef_sets,  f.plan.cdef_select,
                    f.plan.restoration, (leafopt & 4) != 0, s->cfg.intra_edge_filter,
-                   f.fp.frame_is_intra, f.fp.tx_mode_select};
+                   f.fp.frame_is_intra, f.fp.tx_mode_select || f.fp.tx_search}; /* the intra phase's kernel */
   memcpy(g.v, v, sizeof v);
   return g;
 }
