@@ -78,9 +78,9 @@ struct RLds : RCommon {
   /* the level schedule: the block records, per block the dependency level
    * (0: not a small intra block), the BlockDecoded bits its prediction reads
    * (above-right, below-left per plane) and the schedule (small intra blocks
-   * by segment and level); pok: no block is smaller than 8x8 */
+   * by segment and level) */
   Mav1BlockInfo sbb[64];
-  int plv[64], pav[64], pord[64], pok;
+  int plv[64], pav[64], pord[64];
   alignas(4) uint8_t cover[256]; /* per 4x4 cell of the superblock the index of its block */
   SiWave psw[RW];
   int ufl[64];              /* per block: U's CfL alpha is set (V's CfL waits for it) */
@@ -1031,10 +1031,9 @@ DEVI bool wait_flag(const int *flag, int maxSpin) {
 }
 
 /* ---- the level schedule of a superblock ----
- * When no block of a superblock is smaller than 8x8, its small intra blocks
- * (8x8 .. 16x16: one transform block per plane, or with tx_mode_select a
- * luma depth search) are coded by dependency level instead of strictly one
- * after another. A block's level is one more than the highest level of the
+ * A superblock's small intra blocks (8x8 .. 16x16: one transform block per
+ * plane, or with tx_mode_select a luma depth search) are coded by dependency
+ * level instead of strictly one after another. A block's level is one more than the highest level of the
  * earlier (decode order) intra blocks of the superblock that its prediction
  * may read: those covering the column left of it down to twice its height,
  * the row above it right to twice its width, or the corner; blocks of one
@@ -1042,17 +1041,18 @@ DEVI bool wait_flag(const int *flag, int maxSpin) {
  * reads (above-right, below-left, per plane) are those of decode order: the
  * superblock's initial flags, or set where an earlier block of the
  * superblock covers the cell (the cover map: per 4x4 luma cell the index of
- * its block; a chroma cell is its top left luma cell's, as no block is
- * smaller than 8x8). Covering whole blocks equals marking their transform
+ * its block; a chroma cell counts as its top left luma cell: where blocks
+ * below 8x8 share it, that is the first of them, and each of them codes and
+ * marks the whole cell). Covering whole blocks equals marking their transform
  * blocks inside the frame, and a cell outside the frame never changes a
  * prediction (the edge fetch clamps to the frame).
- * Larger intra blocks cut the superblock into segments: the small blocks
+ * The other intra blocks (larger than 16x16, 4:1, or below 8x8, which the
+ * analysis never chooses) cut the superblock into segments: the small blocks
  * before one are finished, the whole workgroup codes it, and the schedule
  * goes on behind it; levels count within a segment only.
  * The blocks run as a dataflow over these dependencies (lvl_dataflow below);
  * the level pass records per block the mask of the earlier intra blocks it
- * reads (dmask). In a superblock with a smaller block (which the analysis
- * never chooses) or without loss every intra block counts as larger. */
+ * reads (dmask). Without loss no block is small. */
 /* Whether block i's BlockDecoded flag of plane p's 4x4 cell (y, x) of the
  * superblock is set when its turn comes in decode order. */
 DEVI int lvl_decoded(int i, int p, int y, int x) {
@@ -1078,7 +1078,7 @@ DEVI void lvl_schedule(const Mav1FrameParams &fp, int n) {
   for (int q = tid; q < n * 6; q += RT) {
     const int i = q / 6, p = (q >> 1) % 3, f = q & 1, sub = p > 0;
     const Mav1BlockInfo &b = L.sbb[i];
-    if (!(L.pok && si_small(fp, b))) continue;
+    if (!si_small(fp, b)) continue;
     const int txSz = p ? uv_tx_size(b.bsize) : Max_Tx_Size_Rect[b.bsize];
     const int stepX = Tx_Width[txSz] >> 2, stepY = Tx_Height[txSz] >> 2;
     const int by = (b.mi_row & 15) >> sub, bx = (b.mi_col & 15) >> sub;
@@ -1088,7 +1088,7 @@ DEVI void lvl_schedule(const Mav1FrameParams &fp, int n) {
     for (int q = tid; q < n * 8; q += RT) {
       const int i = q >> 3, f = (q >> 2) & 1, k = (q & 3) + 1;
       const Mav1BlockInfo &b = L.sbb[i];
-      if (!L.pok || !si_small(fp, b) || k > (f ? Num_4x4_Blocks_High[b.bsize] : Num_4x4_Blocks_Wide[b.bsize])) continue;
+      if (!si_small(fp, b) || k > (f ? Num_4x4_Blocks_High[b.bsize] : Num_4x4_Blocks_Wide[b.bsize])) continue;
       const int by = b.mi_row & 15, bx = b.mi_col & 15;
       if (lvl_decoded(i, 0, f ? by + k : by - 1, f ? bx - 1 : bx + k)) atomicOr(&L.pavl[i], 1 << (8 * f + k));
     }
@@ -1103,7 +1103,7 @@ DEVI void lvl_schedule(const Mav1FrameParams &fp, int n) {
       hj = Num_4x4_Blocks_High[o.bsize];
       wj = Num_4x4_Blocks_Wide[o.bsize];
       intraJ = !o.is_inter;
-      smallJ = L.pok && si_small(fp, o);
+      smallJ = si_small(fp, o);
     }
     const unsigned long long big = __ballot(intraJ && !smallJ);
     const int segJ = __popcll(big & ((1ull << j) - 1));
@@ -1532,8 +1532,7 @@ DEVI void intra_sb_prep(const Mav1FrameParams &fp, const Mav1BlockInfo *__restri
       ts[q] = *(const uint32_t *)(src + fp.offset[p] + Y * stride + X);
     }
   }
-  /* the block records; the level schedule applies when no block is smaller
-   * than 8x8 */
+  /* the block records */
   const int nb = S.num_blocks;
   for (int q = tid; q < nb * 27; q += RT) ((int32_t *)L.sbb)[q] = ((const int32_t *)(blocks + S.first_block))[q];
   for (int q = tid; q < 64; q += RT) {
@@ -1546,14 +1545,8 @@ DEVI void intra_sb_prep(const Mav1FrameParams &fp, const Mav1BlockInfo *__restri
     L.rrel[tid] = -1;
   }
   if (tid == 0) {
-    L.pok = !fp.lossless;
     L.lerr = 0;
     L.ldm = L.udm = L.vdm = 0;
-  }
-  __syncthreads();
-  if (tid < nb) {
-    const int bs = L.sbb[tid].bsize;
-    if (bs < BLOCK_8X8 || bs == BLOCK_4X16 || bs == BLOCK_16X4) L.pok = 0;
   }
   __syncthreads();
   lvl_schedule(fp, nb);
