@@ -454,7 +454,7 @@ hipError_t launch_recon_intra_plain_b(hipStream_t st, const BatchFrame *T, int n
 hipError_t launch_recon_intra_search_b(hipStream_t st, const BatchFrame *T, int n, int *q, int workgroups);
 
 /* Whether the frame's intra luma blocks search transform types or depths. */
-static bool intra_search(const Mav1FrameParams &fp) { return fp.tx_mode_select || fp.tx_search; }
+__host__ DEVI bool intra_search(const Mav1FrameParams &fp) { return fp.tx_mode_select || fp.tx_search; }
 
 hipError_t launch_recon_intra(hipStream_t st, const Mav1FrameParams &fp, Mav1BlockInfo *blocks, const Mav1SbInfo *sbs,
                               const uint8_t *src, uint8_t *rec, const uint8_t *ref, const uint8_t *gold,
@@ -463,15 +463,20 @@ hipError_t launch_recon_intra(hipStream_t st, const Mav1FrameParams &fp, Mav1Blo
                                                                                    gold, coefs, mats, iwork, workgroups);
 }
 
-hipError_t launch_recon_intra_b(hipStream_t st, const BatchFrame *T, const BatchFrame *H, int n, int *q,
-                                int workgroups) {
-  /* the frames of a round agree on the search */
-  for (int f = 1; f < n; f++)
-    if (intra_search(H[f].fp) != intra_search(H[0].fp)) return hipErrorInvalidValue;
-  return (intra_search(H[0].fp) ? launch_recon_intra_search_b : launch_recon_intra_plain_b)(st, T, n, q, workgroups);
-}
-
 #include "recon_queue.h"
+
+size_t intra_queue_ints(int qcap) { return 2 * (size_t)QH_INTS(qcap); }
+
+int intra_searches(const BatchFrame *H, int n) {
+  int search = 0;
+  for (int f = 0; f < n; f++) search += intra_search(H[f].fp);
+  return search;
+}
+hipError_t launch_recon_intra_b(hipStream_t st, const BatchFrame *T, int n, int *q, int qcap, int search,
+                                int workgroups) {
+  return search ? launch_recon_intra_search_b(st, T, n, q + QH_INTS(qcap), workgroups)
+                : launch_recon_intra_plain_b(st, T, n, q, workgroups);
+}
 
 /* ---- batched launches (batch.h): the same kernels over several frames ---- */
 
@@ -534,17 +539,19 @@ __global__ __launch_bounds__(SCHED_T) void k_intra_sched_b(const BatchFrame *__r
 }
 
 __global__ void k_intra_queue_reset_b(int *__restrict__ q, int cap) {
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < cap; i += gridDim.x * blockDim.x) q[QH_ITEMS + i] = -1;
-  if (blockIdx.x == 0 && threadIdx.x < QH_ITEMS) q[threadIdx.x] = 0;
+  const int n = QH_INTS(cap);
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+    q[i] = q[n + i] = i < QH_ITEMS ? 0 : -1;
 }
 
 /* Per frame (one workgroup each, after the scheduling pass): the pending
  * dependency count of every superblock holding intra blocks; those with none
- * are queued. */
-__global__ __launch_bounds__(256) void k_intra_ready_b(const BatchFrame *__restrict__ T, int *__restrict__ q) {
+ * are queued, in the queue of the frame's intra kernel. */
+__global__ __launch_bounds__(256) void k_intra_ready_b(const BatchFrame *__restrict__ T, int *__restrict__ q, int qcap) {
   const int f = blockIdx.x;
   const BatchFrame &F = T[f];
   const Mav1FrameParams &fp = F.fp;
+  if (intra_search(fp)) q += QH_INTS(qcap);
   const int n = fp.sb_cols * fp.sb_rows;
   const int *has = gptr(F.iwork) + IW_HDR + n;
   int *cnt = gptr(F.iwork) + IW_HDR + 3 * n;
@@ -585,7 +592,7 @@ hipError_t launch_intra_sched_b(hipStream_t st, const BatchFrame *T, const Batch
   for (int f = 0; f < n; f++) need += H[f].fp.sb_cols * H[f].fp.sb_rows;
   if (need > qcap || n > (1 << 14)) return hipErrorInvalidValue;
   hipLaunchKernelGGL(k_intra_sched_b, dim3(n), dim3(SCHED_T), 0, st, T);
-  hipLaunchKernelGGL(k_intra_queue_reset_b, dim3(std::min((qcap + 255) / 256, 1024)), dim3(256), 0, st, q, qcap);
-  hipLaunchKernelGGL(k_intra_ready_b, dim3(n), dim3(256), 0, st, T, q);
+  hipLaunchKernelGGL(k_intra_queue_reset_b, dim3(std::min((QH_INTS(qcap) + 255) / 256, 1024)), dim3(256), 0, st, q, qcap);
+  hipLaunchKernelGGL(k_intra_ready_b, dim3(n), dim3(256), 0, st, T, q, qcap);
   return hipGetLastError();
 }

@@ -15,11 +15,14 @@
  * the entries ((frame << 16) | superblock, -1 until filled). Every entry is
  * filled once all superblocks before it in dependency order are done, so a
  * workgroup's wait for its entry ends; the wait is still bounded, and one
- * that runs out sets every frame's error word. */
+ * that runs out sets every frame's error word.
+ * A batch has two queues, one behind the other: of the frames without a luma
+ * search and of those with one, whose intra kernels differ. */
 #define QH_HEAD 0
 #define QH_TAIL 1
 #define QH_TOTAL 2
 #define QH_ITEMS 4
+#define QH_INTS(cap) (QH_ITEMS + (cap)) /* of one queue with room for cap superblocks */
 
 /* The superblocks whose reconstruction superblock sb reads (-1: none), as
  * the single-frame intra phase waits for them. */

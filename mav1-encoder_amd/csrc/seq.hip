@@ -832,7 +832,7 @@ Sig sig_of(const mav1hip_seq *s, const Frame &f) {
                    f.fp.golden,        f.fp.turbo,        f.plan.filter_info,
                    f.plan.deblock,     f.plan.cdef_sets,  f.plan.cdef_select,
                    f.plan.restoration, (leafopt & 4) != 0, s->cfg.intra_edge_filter,
-                   f.fp.frame_is_intra, f.fp.tx_mode_select || f.fp.tx_search}; /* the intra phase's kernel */
+                   f.fp.frame_is_intra};
   memcpy(g.v, v, sizeof v);
   return g;
 }
@@ -942,7 +942,23 @@ int round_late(mav1hip_batch *b, Round &R) {
   const bool intraFrame = R.frames[0].fp.frame_is_intra != 0;
   int intraWg = intraFrame ? b->intra_wg_key : b->intra_wg_inter;
   if (intraWg <= 0) intraWg = intraFrame ? b->num_cu : std::max(1, b->num_cu / 4);
-  LCHK(b, "recon_intra", launch_recon_intra_b(st, T, H, n, b->d_iq[e], intraWg));
+  /* Streams with and without a luma search share the round, and their intra
+   * phases, two kernels, run side by side. Half of the streams with a type
+   * search, 5 frames each: eight of 204x116 5.9 ms, four of 1920x1080 40.8 ms;
+   * with a round for each kind, which launches every stage twice, 8.0 and
+   * 46.0 ms, with the kernels one after the other 7.1 and 47.0 ms. */
+  const int search = intra_searches(H, n);
+  hipStream_t sst = search < n ? ctx_side_stream(s0->eng[e].ctx) : st;
+  if (search && search < n) {
+    BCHK(b, hipEventRecord(b->me_done[e][0], st));
+    BCHK(b, hipStreamWaitEvent(sst, b->me_done[e][0], 0));
+  }
+  if (search) LCHK(b, "recon_intra", launch_recon_intra_b(sst, T, n, b->d_iq[e], b->iq_cap, 1, intraWg));
+  if (search < n) LCHK(b, "recon_intra", launch_recon_intra_b(st, T, n, b->d_iq[e], b->iq_cap, 0, intraWg));
+  if (search && search < n) {
+    BCHK(b, hipEventRecord(b->ana_done[e], sst));
+    BCHK(b, hipStreamWaitEvent(st, b->ana_done[e], 0));
+  }
   const Frame &f0 = R.frames[0];
   const Mav1HipFilterPlan &pl = f0.plan;
   if (pl.filter_info) {
@@ -1059,7 +1075,7 @@ int batch_setup(mav1hip_batch *b) {
   }
   b->num_cu = ctx_num_cu(b->seqs[0]->eng[0].ctx);
   for (auto *s : b->seqs) b->iq_cap += s->num_sbs;
-  for (auto &q : b->d_iq) BCHK(b, hipMalloc((void **)&q, sizeof(int) * (4 + (size_t)b->iq_cap)));
+  for (auto &q : b->d_iq) BCHK(b, hipMalloc((void **)&q, sizeof(int) * intra_queue_ints(b->iq_cap)));
   return MAV1HIP_OK;
 }
 

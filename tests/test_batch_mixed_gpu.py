@@ -1,6 +1,6 @@
 """A batch whose streams differ in the luma search (transform types, depths or
-neither): their intra phases take different kernels, so their frames go in
-different rounds; equal to each stream's own sequence driver."""
+neither): their frames share the rounds and their intra phases take different
+kernels; equal to each stream's own sequence driver."""
 import pytest
 
 import mav1hip
