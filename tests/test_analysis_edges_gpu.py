@@ -11,7 +11,7 @@ from test_analysis_gpu import run_case
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("w,h,q", [(18, 34, 30), (66, 34, 200), (142, 98, 90), (98, 162, 255)])
+@pytest.mark.parametrize("w,h,q", [(18, 34, 30), (67, 35, 60), (66, 34, 200), (142, 98, 90), (141, 99, 120), (98, 162, 255)])
 @pytest.mark.parametrize("kind", ["key", "inter", "compound"])
 def test_analysis_edges(gpu, w, h, q, kind):
     print(f"[analysis] {w}x{h} q{q} {kind}", flush=True)
