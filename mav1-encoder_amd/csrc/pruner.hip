@@ -781,7 +781,7 @@ struct mav1hip_pruner {
   float *hm = nullptr, *h = nullptr, *logits = nullptr, *dlog = nullptr, *dh = nullptr, *lossb = nullptr;
   float *loss = nullptr, *part = nullptr;
   int slices = 1; /* workgroups of k_forward and k_backward: one per CU */
-  int packed = 0, forwarded = 0, labelled = 0, stored = 0;
+  int packed = 0, forwarded = 0, labelled = 0;
 };
 
 namespace {
@@ -967,9 +967,8 @@ int mav1hip_pruner_forward(mav1hip_pruner *p, float *logits, float *loss) {
   if (!p || p->batch < 1) return pfail(p, MAV1HIP_EINVAL, "forward: no batch loaded");
   int rc;
   if ((rc = pack(p))) return rc;
-  /* the activations are for the backward pass, which without labels is not expected */
+  /* the activations are for the backward pass, whose gradients are zero without labels */
   if ((rc = forward(p, p->labelled))) return rc;
-  p->stored = p->labelled;
   hipLaunchKernelGGL(k_loss_sum, dim3(1), dim3(256), 0, p->st, p->lossb, p->loss, p->batch);
   PCHK(p, hipGetLastError());
   if (logits)
@@ -983,16 +982,15 @@ int mav1hip_pruner_forward(mav1hip_pruner *p, float *logits, float *loss) {
 
 int mav1hip_pruner_backward(mav1hip_pruner *p, float *grads) {
   if (!p || !p->forwarded) return pfail(p, MAV1HIP_EINVAL, "backward: run forward first");
-  int rc;
-  if (!p->stored && (rc = forward(p, true))) return rc;
-  p->stored = 1;
   hipLaunchKernelGGL(k_head_bwd, dim3((p->batch + 3) / 4), dim3(256), 0, p->st, p->logits, p->labels, p->P, p->dlog,
                      p->dh, p->batch);
   hipLaunchKernelGGL(k_head_grads, dim3((NF * NP + NP + NF * NM + NM + 2 * NF + 3) / 4), dim3(256), 0, p->st, p->h,
                      p->q, p->dlog, p->dh, p->G, p->batch);
-  const int n = p->batch < p->slices ? p->batch : p->slices;
-  hipLaunchKernelGGL(k_backward, dim3(n), dim3(PT), 0, p->st, p->x0, p->y1, p->y2, p->y3, p->dh, p->wt2, p->wt3,
-                     p->part, p->batch);
+  /* without labels the forward pass kept no activations: no slices, so the sums are zeros */
+  const int n = !p->labelled ? 0 : p->batch < p->slices ? p->batch : p->slices;
+  if (n)
+    hipLaunchKernelGGL(k_backward, dim3(n), dim3(PT), 0, p->st, p->x0, p->y1, p->y2, p->y3, p->dh, p->wt2, p->wt3,
+                       p->part, p->batch);
   hipLaunchKernelGGL(k_slice_sum, dim3((P_WQ + 63) / 64), dim3(256), 0, p->st, p->part, p->G, n);
   PCHK(p, hipGetLastError());
   if (grads) {

@@ -41,10 +41,14 @@ def test_batch_equals_its_halves(gpu, B):
 
 
 def test_unlabelled_batch_has_zero_gradients(gpu):
-    x, q, _ = batch(np.random.default_rng(7), 5)
+    x, q, labels = batch(np.random.default_rng(7), 5)
     net = mav1hip.Pruner(max_batch=8)
     net.set_params(params(net, 2))
+    logits, _, grads = run(net, x, q, labels)
     net.load(x, q)
     a = net.forward()[0]
-    assert not np.any(net.backward())
+    assert np.array_equal(a, logits)
+    assert np.any(grads) and not np.any(net.backward())
     assert np.array_equal(a, net.forward()[0])
+    # and a labelled batch after it has its own again
+    assert np.array_equal(run(net, x, q, labels)[2], grads)
