@@ -856,6 +856,7 @@ int pruner_infer_frames(mav1hip_pruner *p, hipStream_t st, const BatchFrame *T, 
   hipStream_t own = p->st;
   p->st = st;
   p->batch = total;
+  p->forwarded = 0; /* the loaded batch's inputs and features are overwritten: no backward pass on them */
   int rc = pack(p);
   if (!rc) {
     hipLaunchKernelGGL(k_frame_input, dim3(total), dim3(256), 0, st, T, g, p->x0, p->q);
