@@ -599,8 +599,8 @@ int mav1hip_launch_recon(mav1hip_ctx *c) {
   if (rc) return rc;
   HIPCHK(c, hipStreamWaitEvent(c->stream, c->sched_done, 0));
   return timed(c, "recon_intra", [&] {
-    return launch_recon_intra(c->stream, fp, c->d_blocks, c->d_sbs, c->b_src, c->d_rec, c->b_ref, c->b_gold,
-                              c->d_coefs, c->d_mats, c->d_iwork, intra_workgroups(fp, c->num_cu));
+    return launch_recon_intra(c->stream, fp, c->d_blocks, c->d_sbs, c->b_src, c->d_rec, c->d_coefs, c->d_mats,
+                              c->d_iwork, intra_workgroups(fp, c->num_cu));
   });
 }
 

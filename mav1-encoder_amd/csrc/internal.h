@@ -49,8 +49,8 @@ int intra_workgroups(const Mav1FrameParams &fp, int num_cu);
 hipError_t launch_intra_sched(hipStream_t st, const Mav1FrameParams &fp, const Mav1BlockInfo *blocks,
                               const Mav1SbInfo *sbs, int *iwork);
 hipError_t launch_recon_intra(hipStream_t st, const Mav1FrameParams &fp, Mav1BlockInfo *blocks, const Mav1SbInfo *sbs,
-                              const uint8_t *src, uint8_t *rec, const uint8_t *ref, const uint8_t *gold,
-                              int32_t *coefs, const int32_t *mats, int *iwork, int workgroups);
+                              const uint8_t *src, uint8_t *rec, int32_t *coefs, const int32_t *mats, int *iwork,
+                              int workgroups);
 
 /* filters.hip */
 hipError_t launch_filter_info(hipStream_t st, const Mav1FrameParams &fp, const Mav1BlockInfo *blocks,

@@ -21,6 +21,7 @@
  * three shared horizontal passes. Larger transforms (32- and 64-point) use
  * the whole workgroup per candidate. */
 #include "recon_lds.h"
+#include "recon_queue.h"
 
 /* Inter prediction: the reference window and the horizontal pass of up to
  * three filters; compound: the first prediction and a band of the second. */
@@ -440,30 +441,15 @@ hipError_t launch_intra_sched(hipStream_t st, const Mav1FrameParams &fp, const M
   return hipGetLastError();
 }
 
-/* ---- the intra phase's launchers: recon_intra.hip (no luma search),
- * recon_search.hip (transform type or depth search) ---- */
-hipError_t launch_recon_intra_plain(hipStream_t st, const Mav1FrameParams &fp, Mav1BlockInfo *blocks,
-                                    const Mav1SbInfo *sbs, const uint8_t *src, uint8_t *rec, const uint8_t *ref,
-                                    const uint8_t *gold, int32_t *coefs, const int32_t *mats, int *iwork,
-                                    int workgroups);
-hipError_t launch_recon_intra_search(hipStream_t st, const Mav1FrameParams &fp, Mav1BlockInfo *blocks,
-                                     const Mav1SbInfo *sbs, const uint8_t *src, uint8_t *rec, const uint8_t *ref,
-                                     const uint8_t *gold, int32_t *coefs, const int32_t *mats, int *iwork,
-                                     int workgroups);
-hipError_t launch_recon_intra_plain_b(hipStream_t st, const BatchFrame *T, int n, int *q, int workgroups);
-hipError_t launch_recon_intra_search_b(hipStream_t st, const BatchFrame *T, int n, int *q, int workgroups);
-
 /* Whether the frame's intra luma blocks search transform types or depths. */
 __host__ DEVI bool intra_search(const Mav1FrameParams &fp) { return fp.tx_mode_select || fp.tx_search; }
 
 hipError_t launch_recon_intra(hipStream_t st, const Mav1FrameParams &fp, Mav1BlockInfo *blocks, const Mav1SbInfo *sbs,
-                              const uint8_t *src, uint8_t *rec, const uint8_t *ref, const uint8_t *gold,
-                              int32_t *coefs, const int32_t *mats, int *iwork, int workgroups) {
-  return (intra_search(fp) ? launch_recon_intra_search : launch_recon_intra_plain)(st, fp, blocks, sbs, src, rec, ref,
-                                                                                   gold, coefs, mats, iwork, workgroups);
+                              const uint8_t *src, uint8_t *rec, int32_t *coefs, const int32_t *mats, int *iwork,
+                              int workgroups) {
+  return (intra_search(fp) ? launch_recon_intra_search : launch_recon_intra_plain)(st, fp, blocks, sbs, src, rec, coefs,
+                                                                                   mats, iwork, workgroups);
 }
-
-#include "recon_queue.h"
 
 size_t intra_queue_ints(int qcap) { return 2 * (size_t)QH_INTS(qcap); }
 

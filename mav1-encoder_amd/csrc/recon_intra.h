@@ -910,24 +910,21 @@ DEVI SiGeo si_geo(const Mav1BlockInfo &b, int plane) {
 }
 
 /* Prediction of one plane of small block b by one wave (code_plane's
- * intra_tx_predict call); for CfL also the alphas' SSEs (cfl_tx), and for U
- * the chosen alpha applied. */
-DEVI void si_predict(const Mav1FrameParams &fp, Mav1BlockInfo &b, int plane, SiWave &W, int har = -1, int hbl = -1,
-                     int cflW = -1, int cflH = -1) {
+ * intra_tx_predict call) with its BlockDecoded bits above right (har) and
+ * below left (hbl); for CfL also the alphas' SSEs (cfl_tx), with the end of
+ * the coded luma (cflW, cflH; -1: the block's one transform block). */
+DEVI void si_predict(const Mav1FrameParams &fp, Mav1BlockInfo &b, int plane, SiWave &W, int har, int hbl, int cflW = -1,
+                     int cflH = -1) {
   const TxCtx c = wave_ctx();
   const int lane = c.tid;
   const SiGeo g = si_geo(b, plane);
   plane = d_uni(plane);
-  const int sub = g.sub, stepX = d_uni(Tx_Width[g.txSz]) >> 2, stepY = d_uni(Tx_Height[g.txSz]) >> 2;
-  const int sbr = ((g.sy << sub) >> 2) & 15, sbc = ((g.sx << sub) >> 2) & 15;
-  const int mr = d_uni(b.mi_row), mc = d_uni(b.mi_col);
+  const int sub = g.sub, mr = d_uni(b.mi_row), mc = d_uni(b.mi_col);
   const int availU = mr > 0, availL = mc > tile_start(fp, mc);
   const int uvMode = d_uni(b.uv_mode);
   const int isCfl = plane > 0 && uvMode == UV_CFL_PRED;
   wave_predict(g.px, g.S, g.sx, g.sy, g.lw, g.lh, d_uni(plane == 0 ? b.y_mode : (isCfl ? DC_PRED : uvMode)),
-                   d_uni(plane == 0 ? b.angle_y : b.angle_uv), availL, availU,
-                   d_uni(har >= 0 ? har : gL.bd[BDI(plane, (sbr >> sub) - 1, (sbc >> sub) + stepX)]),
-                   d_uni(hbl >= 0 ? hbl : gL.bd[BDI(plane, (sbr >> sub) + stepY, (sbc >> sub) - 1)]),
+                   d_uni(plane == 0 ? b.angle_y : b.angle_uv), availL, availU, har, hbl,
                    ((fp.mi_cols * 4) >> sub) - 1, ((fp.mi_rows * 4) >> sub) - 1, fp.enable_intra_edge_filter,
                    d_uni((b.interp_filter >> (plane == 0 ? 4 : 5)) & 1), W);
   if (!isCfl) return;
@@ -1193,12 +1190,16 @@ DEVI void lvl_publish(unsigned long long *m, int i) {
  * depths run side by side, each in a private copy of the block (RdDeep /
  * RdShallow); the cheapest (the shallowest on a tie) goes into the tile. The
  * deepest depth of every small block is 4x4.
- * Bound by the serial chain of 4x4 blocks (prediction, then search) on the
- * deepest depth's wave. Coding each transform block by the whole workgroup
- * took about 30k cycles with its five barriers (11.3M per superblock); two
- * waves per block and one block per team let independent blocks, depths and
- * chroma run side by side: five full-RD frames of 1280x720 took 289 ms, with
- * this split 80 ms, with the waves' transforms in registers 62 ms. */
+ * Bound by the serial chain of prediction and search on the longer wave. For
+ * a 16x16 block that is the shallower depths' one: 86k cycles for the types of
+ * the 16x16 transform, one after the other, and about 11k for each 8x8 block,
+ * 130k in all, against 85k for the sixteen 4x4 blocks; for an 8x8 block it is
+ * the deepest depth's one, 21k against 11k. Coding each transform block by
+ * the whole workgroup took about 30k cycles with its five barriers (11.3M per
+ * superblock); two waves per block and one block per team let independent
+ * blocks, depths and chroma run side by side: five full-RD frames of 1280x720
+ * took 289 ms, with this split 80 ms, with the waves' transforms in registers
+ * 62 ms. */
 
 /* The private pixel copy addressed by plane position, for the block at luma
  * (x0, y0). */
@@ -1228,8 +1229,7 @@ DEVI RdRes rd_depth(const Mav1FrameParams &fp, const Mav1BlockInfo &b, int depth
    * then the left column to twice the height (inside the tile; rows below
    * it are never read) */
   {
-    const int nc = 2 * n4w + 1, w = n4w * 4, h = n4h * 4, cx = lane & 15, bottom = (mr | 15) * 4 + 3;
-    (void)w;
+    const int nc = 2 * n4w + 1, h = n4h * 4, cx = lane & 15, bottom = (mr | 15) * 4 + 3;
     if (cx < nc)
       for (int rr = (lane >> 4) - 1; rr < h; rr += 4)
         *(lds_u32 *)(px + (y0 + rr) * RD_PS + x0 - 4 + 4 * cx) =
@@ -1449,8 +1449,7 @@ DEVI void lvl_dataflow(const Mav1FrameParams &fp, int32_t *__restrict__ coefs, c
         const int eob = tx_eval<true>(c, fp, g.spx, g.S, g.px, g.S, g.sx, g.sy, g.txSz, 0, DCT_DCT, true, W.resid, SRS,
                                       W.tmp, W.coef, W.q, W.dq, SQS, mats, &cost);
         /* the reconstruction first: the blocks waiting for this one read only
-         * its pixels; then the levels out and the block's transform fields
-         * (lvl_luma_out's work, in that order) */
+         * its pixels; then the levels out and the block's transform fields */
         if (eob > 0)
           wave_recon_any(c, W.q, W.resid, g.txSz, DCT_DCT, fp.dc_q[0], fp.ac_q[0], g.px, g.S, g.sx, g.sy);
         lvl_publish(&L.ldm, i);
@@ -1510,9 +1509,8 @@ DEVI void intra_sb_prep(const Mav1FrameParams &fp, const Mav1BlockInfo *__restri
                         const uint8_t *__restrict__ src, int r, int c) {
   RLds &L = gL;
   const int tid = threadIdx.x;
-  const int c0 = 0, cl = c;
   /* clear_block_decoded_flags (k_recon.h:402-414) */
-  const int mr = r * 16, mc = (c0 + cl) * 16;
+  const int mr = r * 16, mc = c * 16;
   const int tileEnd = d_min(fp.mi_cols, tile_start(fp, mc) + fp.tile_w_sb * 16);
   for (int q = tid; q < 3 * BDD * BDD; q += RT) {
     const int p = q / (BDD * BDD), e = q - p * BDD * BDD, y = e / BDD - 1, x = e % BDD - 1, sub = p > 0;
@@ -1524,7 +1522,7 @@ DEVI void intra_sb_prep(const Mav1FrameParams &fp, const Mav1BlockInfo *__restri
   /* the superblock's source tile, as dwords */
   for (int p = 0; p < 3; p++) {
     const int sub = p > 0, TS = sub ? TS_C : TS_Y, n = 64 >> sub, wpr = TS / 4;
-    const int oy = ((r * 64) >> sub) - 1, ox = (((c0 + cl) * 64) >> sub) - 4, stride = fp.stride[p];
+    const int oy = ((r * 64) >> sub) - 1, ox = ((c * 64) >> sub) - 4, stride = fp.stride[p];
     uint32_t *ts = (uint32_t *)(L.tile[1] + (p == 0 ? 0 : TILE_Y + (p - 1) * TILE_C));
     for (int q = tid; q < (n + 1) * wpr; q += RT) {
       const int ty = q / wpr, tx = (q - ty * wpr) * 4, Y = oy + ty, X = ox + tx;
@@ -1562,10 +1560,9 @@ DEVI int intra_sb(const Mav1FrameParams &fp, Mav1BlockInfo *__restrict__ blocks,
                   uint8_t *rec, int32_t *__restrict__ coefs, const int32_t *__restrict__ mats, int r, int c) {
   RLds &L = gL;
   const int tid = threadIdx.x;
-  const int c0 = 0, cl = c;
   for (int p = 0; p < 3; p++) {
     const int sub = p > 0, TS = sub ? TS_C : TS_Y, n = 64 >> sub, wpr = TS / 4;
-    const int oy = ((r * 64) >> sub) - 1, ox = (((c0 + cl) * 64) >> sub) - 4, stride = fp.stride[p];
+    const int oy = ((r * 64) >> sub) - 1, ox = ((c * 64) >> sub) - 4, stride = fp.stride[p];
     uint32_t *tr = (uint32_t *)(L.tile[0] + (p == 0 ? 0 : TILE_Y + (p - 1) * TILE_C));
     for (int q = tid; q < (n + 1) * wpr; q += RT) {
       const int ty = q / wpr, tx = (q - ty * wpr) * 4, Y = oy + ty, X = ox + tx;
@@ -1605,7 +1602,7 @@ DEVI int intra_sb(const Mav1FrameParams &fp, Mav1BlockInfo *__restrict__ blocks,
   /* the superblock back into the frame */
   for (int p = 0; p < 3; p++) {
     const int sub = p > 0, TS = sub ? TS_C : TS_Y, n = 64 >> sub, wpr = n / 4;
-    const int y0 = (r * 64) >> sub, x0 = ((c0 + cl) * 64) >> sub, stride = fp.stride[p];
+    const int y0 = (r * 64) >> sub, x0 = (c * 64) >> sub, stride = fp.stride[p];
     const uint32_t *tr = (const uint32_t *)(L.tile[0] + (p == 0 ? 0 : TILE_Y + (p - 1) * TILE_C));
     for (int q = tid; q < n * wpr; q += RT) {
       const int ty = q / wpr, tx = (q - ty * wpr) * 4;

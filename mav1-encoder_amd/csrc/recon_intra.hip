@@ -3,11 +3,8 @@
 #include "recon_intra.h"
 
 hipError_t launch_recon_intra_plain(hipStream_t st, const Mav1FrameParams &fp, Mav1BlockInfo *blocks,
-                                 const Mav1SbInfo *sbs, const uint8_t *src, uint8_t *rec, const uint8_t *ref,
-                                 const uint8_t *gold, int32_t *coefs, const int32_t *mats, int *iwork,
-                                 int workgroups) {
-  (void)ref;
-  (void)gold;
+                                    const Mav1SbInfo *sbs, const uint8_t *src, uint8_t *rec, int32_t *coefs,
+                                    const int32_t *mats, int *iwork, int workgroups) {
   hipLaunchKernelGGL(k_recon_intra<false>, dim3(workgroups), dim3(RT), 0, st, fp, blocks, sbs, src, rec, coefs, mats,
                      iwork, 1 << 20);
   return hipGetLastError();

@@ -1,9 +1,22 @@
-/* The batched intra phase's ready queue (recon.hip fills it, recon_intra.h
- * takes from it). */
+/* Between recon.hip and the intra phase's kernels: the launchers, and the
+ * batched form's ready queue (recon.hip fills it, recon_intra.h takes from
+ * it). */
 #ifndef MAV1_RECON_QUEUE_H
 #define MAV1_RECON_QUEUE_H
 
 #include "dev_common.h"
+#include "internal.h"
+
+/* Of frames without a luma search (recon_intra.hip) and with a transform type
+ * or depth search (recon_search.hip). */
+hipError_t launch_recon_intra_plain(hipStream_t st, const Mav1FrameParams &fp, Mav1BlockInfo *blocks,
+                                    const Mav1SbInfo *sbs, const uint8_t *src, uint8_t *rec, int32_t *coefs,
+                                    const int32_t *mats, int *iwork, int workgroups);
+hipError_t launch_recon_intra_search(hipStream_t st, const Mav1FrameParams &fp, Mav1BlockInfo *blocks,
+                                     const Mav1SbInfo *sbs, const uint8_t *src, uint8_t *rec, int32_t *coefs,
+                                     const int32_t *mats, int *iwork, int workgroups);
+hipError_t launch_recon_intra_plain_b(hipStream_t st, const BatchFrame *T, int n, int *q, int workgroups);
+hipError_t launch_recon_intra_search_b(hipStream_t st, const BatchFrame *T, int n, int *q, int workgroups);
 
 /* Intra phase over several frames: a dataflow queue. A superblock holding
  * intra blocks enters the batch's ready queue when the last of its
