@@ -10,16 +10,18 @@ import libs
 import mav1hip
 
 needs_ref = pytest.mark.skipif(not libs.ref_available(), reason="oracle/_ref not built (no reference sources)")
+CODER = "ref" if libs.ref_available() else "oracle"  # makes the frames
 
 
 def coded_frame(w, h, kind, seed, turbo=1, **kw):
-    """A frame reconstructed by the reference (ME, analysis, recon), the
-    oracle's filter info of it, and the source."""
+    """A frame reconstructed by the reference, or without its sources by the
+    oracle (ME, analysis, recon), the oracle's filter info of it, and the
+    source."""
     cfg = mav1hip.default_config(w, h, turbo=turbo, qindex=kw.pop("q", 125), **kw)
     fr = mav1hip.turbo_frame(kind, 1) if kind in ("key", "arf", "leaf") else mav1hip.frame_info(order_hint=1, gold_differs=1)
     fp, npresets = mav1hip.setup_params(cfg, fr)
     geo, frames = libs.make_sequence(w, h, 3, seed, n_objects=8, max_vel=10)
-    r = libs.Impl("ref")
+    r = libs.Impl(CODER)
     n = fp.sb_cols * fp.sb_rows * 170
     mvf, mvg = np.zeros(n, np.int32), np.zeros(n, np.int32)
     if not fp.frame_is_intra:
@@ -28,7 +30,8 @@ def coded_frame(w, h, kind, seed, turbo=1, **kw):
     _, _, blocks, sbs = r.analyze(fp, frames[1], frames[0], frames[2], mvf, mvg)
     if cfg.intra_edge_filter:
         blocks = libs.edge_types(libs.Impl("oracle"), fp, blocks, sbs)
-    rec, _, blocks = r.recon(fp, blocks, sbs, frames[1], frames[0], frames[2], libs.ref_mats())
+    rec, _, blocks = r.recon(fp, blocks, sbs, frames[1], frames[0], frames[2],
+                             libs.ref_mats() if CODER == "ref" else mav1hip.forward_matrices())
     info = libs.filter_info(fp, blocks, sbs)
     return cfg, fp, npresets, frames[1], rec, blocks, sbs, info
 
@@ -79,7 +82,7 @@ def test_deblock_levels_and_sharpness(sharp):
 
 def _deblocked(name):
     cfg, fp, npresets, src, rec, blocks, sbs, info = frame(name)
-    return fp, src, libs.Filters("ref").loop_filter(fp, rec, info) if libs.ref_available() else None, info
+    return fp, src, libs.Filters(CODER).loop_filter(fp, rec, info), info
 
 
 @needs_ref
@@ -121,8 +124,6 @@ def test_cdef_select_properties():
     (first one on ties), rec holds it over the mi-aligned area and is
     unchanged elsewhere."""
     fp, src, dbk, info = _deblocked("turbo_arf_352x288")
-    if dbk is None:
-        pytest.skip("needs a reconstructed frame")
     rng = np.random.default_rng(4)
     n = 3
     buf = np.stack([dbk, dbk.copy(), dbk.copy()])
