@@ -106,11 +106,11 @@ BH = [4, 8, 4, 8, 16, 8, 16, 32, 16, 32, 64, 32, 64, 128, 64, 128, 16, 4, 32, 8,
 # default run, from the FETCH_SIZE and WRITE_SIZE passes of
 # profiles/recon_intra_1080p_turbo_stream_pmc.md, scaled by the known-size
 # copy's factors there (fetch x1.9992, write x1.0).
-TRAFFIC = {"recon_intra": 4254069}
+TRAFFIC = {"recon_intra": 3983601}
 # VALUBusy (%) per launch over the timed stream, from the counter pass of the
 # same summary (100 * SQ_ACTIVE_INST_VALU / CU_NUM / GRBM_GUI_ACTIVE).
-VALU_BUSY = {"recon_intra": 0.09, "lr_fit": 6.78, "recon_inter": 2.22, "me_level0": 5.06, "me_level2": 6.89,
-             "me_level3": 8.40, "analyze_level0": 3.10, "qpel_build": 6.53, "cdef": 7.43}
+VALU_BUSY = {"recon_intra": 0.09, "lr_fit": 6.76, "recon_inter": 2.22, "me_level0": 5.03, "me_level2": 6.93,
+             "me_level3": 8.42, "analyze_level0": 3.07, "qpel_build": 6.56, "cdef": 7.45}
 
 
 def intra_phase_bytes(fp, blocks, sbs):
